@@ -158,16 +158,15 @@ __device__ __forceinline__ typename V4<T>::type ld16(const T *P)
 	return acc;
 }
 
-// 1/sqrt(d) to full precision: the hardware estimate refined by Newton
-// steps r <- r + r (1/2 - (d/2) r^2), each doubling the correct bits (two
-// for double, one for float).
+// 1/sqrt(d) to full precision: the hardware estimate r (about 24 bits in
+// either type) and e = 1 - d r^2; for double one third-order step
+// r + r e (1/2 + 3/8 e), whose error is of order e^3, for float one Newton
+// step.
 __device__ __forceinline__ double rsqrt_nr(double d)
 {
-	double r = __builtin_amdgcn_rsq(d);
-	const double h = 0.5 * d;
-	r = fma(r, fma(-h * r, r, 0.5), r);
-	r = fma(r, fma(-h * r, r, 0.5), r);
-	return r;
+	const double r = __builtin_amdgcn_rsq(d);
+	const double e = fma(-d * r, r, 1.0);
+	return fma(r * e, fma(0.375, e, 0.5), r);
 }
 
 __device__ __forceinline__ float rsqrt_nr(float d)
@@ -177,89 +176,125 @@ __device__ __forceinline__ float rsqrt_nr(float d)
 	return fmaf(r, fmaf(-h * r, r, 0.5f), r);
 }
 
+// The hardware estimate of 1/d, and x / d from such an estimate y and
+// e = 1 - d y: x y (1 + e + e^2) for double (error of order e^3), x y (1 + e)
+// for float.
+__device__ __forceinline__ double rcp_est(double d) { return __builtin_amdgcn_rcp(d); }
+__device__ __forceinline__ float rcp_est(float d) { return __builtin_amdgcn_rcpf(d); }
+
+__device__ __forceinline__ double quot_nr(double x, double d, double y)
+{
+	const double e = fma(-d, y, 1.0), x0 = x * y;
+	return fma(x0, fma(e, e, e), x0);
+}
+
+__device__ __forceinline__ float quot_nr(float x, float d, float y)
+{
+	const float e = fmaf(-d, y, 1.0f), x0 = x * y;
+	return fmaf(x0, e, x0);
+}
+
 // Lane t < 16 holds row t of a 16x16 lower block in x[0..15] (columns
-// above the diagonal are ignored).  In-place Cholesky; returns the 1-based
-// index of the first non-positive pivot, or 0.  Each column costs one
-// reciprocal square root (L(k,k) = d * d^{-1/2}, multipliers scaled by
-// d^{-1/2}) instead of a square root and a division.  The pivots and
-// multipliers are broadcast with v_readlane: the row-broadcast DPP form gave
-// a wrong factor here (a 17x17 input) although the same loop in isolation
-// was correct, so this chain stays on the SGPR path.
+// above the diagonal are ignored), lanes 16..63 up to 48 rows of the panel
+// below it.  In-place Cholesky of the block, the panel rows solved against
+// it on the way (the other lanes run the same instructions anyway); returns
+// the 1-based index of the first non-positive pivot, or 0.  The chain from
+// one pivot d to the next is kept short: the columns to the right take
+// x_j -= (x_k / d) x_jk with the unscaled multipliers x_jk, which are
+// broadcast while the quotient is formed; the column itself is scaled by
+// d^{-1/2} off that chain.  The broadcasts are v_readlane: the row-broadcast
+// DPP form reaches only the lanes of one 16-lane row.
 template <typename T>
 __device__ __forceinline__ int potrf16_regs(T (&x)[16])
 {
-	const int t = threadIdx.x & 63;
-	int bad = 0;
+	unsigned long long bad = 0;
 #pragma unroll
 	for (int k = 0; k < 16; k++) {
 		const T d = bcast_rl(x[k], k);
-		if (!(d > T(0)) && bad == 0)
-			bad = k + 1;
-		const T r = rsqrt_nr(d);
-		x[k] = (t == k) ? d * r : x[k] * r;
+		const T y = rcp_est(d);
+		__builtin_amdgcn_sched_barrier(0);
+		// all multipliers of the column in scalar registers, behind the
+		// estimate's latency and before the first is used: a readlane's
+		// result may not be read at once
+		T m[16];
 #pragma unroll
 		for (int j = k + 1; j < 16; j++)
-			x[j] -= x[k] * bcast_rl(x[k], j);
+			m[j] = bcast_rl(x[k], j);
+		const T z = quot_nr(x[k], d, y);
+		bad |= __ballot(!(x[k] > T(0))) & (1ull << k);
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int j = k + 1; j < 16; j++)
+			x[j] -= z * m[j];
+		x[k] *= rsqrt_nr(d);
 	}
-	return bad;
+	return __ffsll((long long)bad);
 }
 
-// 1 / L(t,t) for the row t = lane % 16 held in x: one division per lane, all
-// lanes at once (off the dependency chain of the factorisation), so the
-// inverse is the same whether the block was just factored or loaded.
+// Inverse of the factored 16x16 lower diagonal block J of S into the same
+// block of Li (zeros above its diagonal), by one wave: lane c (mod 16) takes
+// column c.  One division per lane, all lanes at once, then the columns of L
+// from left to right: y_q = s_q / L(q,q), s_i -= L(i,q) y_q for i > q, whose
+// only chain is one product and one multiply-add per column; L(i,q) is read
+// from LDS as a broadcast, off that chain.  The block may just have been
+// factored or loaded: the inverse has the same bits.
 template <typename T>
-__device__ __forceinline__ T diag_recip(const T (&x)[16])
+__device__ __forceinline__ void inv16(const T *S, int J, T *Li)
 {
-	T dg = T(1);
+	const int lane = threadIdx.x & 63, c = lane & 15;
+	const T *B = S + 16 * J + 16 * J * LD;
+	const T rd = T(1) / B[c + c * LD];
+	T y[16];
 #pragma unroll
-	for (int c = 0; c < 16; c++)
-		dg = (c == (threadIdx.x & 15)) ? x[c] : dg;
-	return T(1) / dg;
-}
-
-// Lane t < 16 holds row t of a factored 16x16 lower L and in rdiag the
-// reciprocal of L(t,t); lane c gets column c of inv(L) in y:
-// y_i = (delta_ic - sum_{q<i} L(i,q) y_q) / L(i,i).
-template <typename T>
-__device__ __forceinline__ void inv16_regs(const T (&x)[16], T rdiag, T (&y)[16])
-{
-	const int c = threadIdx.x & 63;
+	for (int i = 0; i < 16; i++)
+		y[i] = (c == i) ? T(1) : T(0);
 #pragma unroll
-	for (int i = 0; i < 16; i++) {
-		T s = (c == i) ? T(1) : T(0);
+	for (int q = 0; q < 16; q++) {
+		y[q] *= bcast(rd, q);
 #pragma unroll
-		for (int q = 0; q < i; q++)
-			s -= bcast(x[q], i) * y[q];
-		y[i] = s * bcast(rdiag, i);
+		for (int i = q + 1; i < 16; i++)
+			y[i] -= B[i + q * LD] * y[q];
 	}
-}
-
-// Rows of the 16x16 diagonal block J of S into lanes 0..15 (lower part);
-// other lanes get an identity row so that they run the same code.
-template <typename T>
-__device__ __forceinline__ void load_rows16(const T *S, int J, T (&x)[16])
-{
-	const int t = threadIdx.x & 63;
-#pragma unroll
-	for (int c = 0; c < 16; c++)
-		x[c] = (t < 16) ? ((c <= t) ? S[(16 * J + t) + (16 * J + c) * LD] : T(0))
-		                : ((c == (t & 15)) ? T(1) : T(0));
-}
-
-template <typename T>
-__device__ __forceinline__ void store_inv16(T *Li, int J, const T (&y)[16])
-{
-	const int c = threadIdx.x & 63;
-	if (c < 16)
+	if (lane < 16)
 #pragma unroll
 		for (int i = 0; i < 16; i++)
 			Li[(16 * J + i) + (16 * J + c) * LD] = y[i];
+}
+
+// sum_{K=J}^{I-1} L_IK Li_KJ, the product that block (I, J) of the inverse
+// takes before its scaling by -Li_II, in MFMA output layout.
+template <typename T>
+__device__ __forceinline__ typename V4<T>::type inv_sum(const T *S, const T *Li, int I, int J)
+{
+	typename V4<T>::type t = zero4<T>();
+	for (int K = J; K < I; K++)
+		t = mm16_nn(&S[16 * I + 16 * K * LD], &Li[16 * K + 16 * J * LD], t);
+	return t;
+}
+
+template <typename T>
+__device__ __forceinline__ void inv_scale(T *Li, int I, int J, typename V4<T>::type t)
+{
+	st16(&Li[16 * I + 16 * J * LD], mm16_nreg(&Li[16 * I + 16 * I * LD], t, zero4<T>()), T(-1));
+}
+
+// LDS written by other lanes of the same wave is read next: keep the order.
+__device__ __forceinline__ void wave_lds_order()
+{
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // FACTOR: Cholesky of the w x w (w <= 64) lower block D (ld ldd, in place)
 // and its inverse into Dinv (64 x 64, ld 64, identity past w).
 // !FACTOR: D is already factored; only the inverse is formed.
 // One 256-thread workgroup; S and Li are two LDS blocks of 64 * LD elements.
+// Bound: the 64 dependent columns.  Wave 0 runs them as four panels of 16
+// columns over all the rows below (potrf16_regs), and everything else
+// overlaps the next panel: the trailing blocks, the 16x16 inverses and the
+// columns of the inverse, one per wave.  Only the update of the next 16
+// columns stands between two panels.
 // Returns, in every thread of wave 0, the 1-based column of the first
 // non-positive pivot within the block (or 0); other threads return 0.
 // Ends with a workgroup barrier, so the caller may reuse S and Li.
@@ -289,70 +324,100 @@ __device__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__rest
 
 	int bad = 0;
 	if (FACTOR) {
+		// wave q = 1..3 keeps the sum of the next block of its inverse column
+		V t = zero4<T>();
+		const int Jc = wave - 1;
+#pragma unroll
 		for (int J = 0; J < 4; J++) {
 			if (wave == 0) {
-				T x[16], y[16];
-				load_rows16(S, J, x);
+				T x[16];
+				const int row = 16 * J + lane;
+#pragma unroll
+				for (int c = 0; c < 16; c++)
+					x[c] = row < 64 ? S[row + (16 * J + c) * LD] : T(0);
 				const int b = potrf16_regs(x);
 				if (b && !bad)
 					bad = 16 * J + b;
-				if (lane < 16)
+				// the diagonal block's upper half, which nothing reads, holds
+				// what the elimination left there
+				if (row < 64)
 #pragma unroll
 					for (int c = 0; c < 16; c++)
-						if (c <= lane)
-							S[(16 * J + lane) + (16 * J + c) * LD] = x[c];
-				inv16_regs(x, diag_recip(x), y);
-				store_inv16(Li, J, y);
+						S[row + (16 * J + c) * LD] = x[c];
+			} else if (J > 0) {
+				// trailing blocks right of column block J, by column block J - 1
+				int p = 0;
+#pragma unroll
+				for (int K = J + 1; K < 4; K++)
+#pragma unroll
+					for (int I = K; I < 4; I++, p++)
+						if (p % 3 == wave - 1) {
+							V acc = ld16(&S[16 * I + 16 * K * LD]);
+							acc = mm16_nt(&S[16 * I + 16 * (J - 1) * LD], &S[16 * K + 16 * (J - 1) * LD], acc, T(-1));
+							st16(&S[16 * I + 16 * K * LD], acc, T(1));
+						}
+				// inverse: row J - 2 of the column is scaled now that Li(J-2,J-2)
+				// is there, then the sum for row J - 1; Li(J-1,J-1)
+				if (wave == 3)
+					inv16(S, J - 1, Li);
+				if (Jc < J - 2)
+					inv_scale(Li, J - 2, Jc, t);
+				if (Jc < J - 1) {
+					wave_lds_order();
+					t = inv_sum(S, Li, J - 1, Jc);
+				}
 			}
 			__syncthreads();
-			// panel: L_IJ = A_IJ * inv(L_JJ)^T
+			// column block J + 1 by the panel just factored
 			if (wave < 3 - J) {
 				const int I = J + 1 + wave;
-				const V acc = mm16_nt(&S[16 * I + 16 * J * LD], &Li[16 * J + 16 * J * LD], zero4<T>(), T(1));
-				st16(&S[16 * I + 16 * J * LD], acc, T(1));
+				V acc = ld16(&S[16 * I + 16 * (J + 1) * LD]);
+				acc = mm16_nt(&S[16 * I + 16 * J * LD], &S[16 * (J + 1) + 16 * J * LD], acc, T(-1));
+				st16(&S[16 * I + 16 * (J + 1) * LD], acc, T(1));
 			}
-			__syncthreads();
-			// trailing: A_IK -= L_IJ * L_KJ^T for J < K <= I < 4
-			int p = 0;
-			for (int I = J + 1; I < 4; I++)
-				for (int K = J + 1; K <= I; K++, p++) {
-					if ((p & 3) != wave)
-						continue;
-					V acc = ld16(&S[16 * I + 16 * K * LD]);
-					acc = mm16_nt(&S[16 * I + 16 * J * LD], &S[16 * K + 16 * J * LD], acc, T(-1));
-					st16(&S[16 * I + 16 * K * LD], acc, T(1));
-				}
-			__syncthreads();
+			if (J < 3)
+				__syncthreads();
 		}
+		if (wave == 0) {
+			inv16(S, 3, Li);
+		} else {
+			if (Jc < 2)
+				inv_scale(Li, 2, Jc, t);
+			wave_lds_order();
+			t = inv_sum(S, Li, 3, Jc);
+		}
+		__syncthreads();
+		if (wave > 0)
+			inv_scale(Li, 3, Jc, t);
 	} else {
-		T x[16], y[16];
-		load_rows16(S, wave, x);
-		inv16_regs(x, diag_recip(x), y);
-		store_inv16(Li, wave, y);
+		inv16(S, wave, Li);
 		__syncthreads();
+		if (wave > 0)
+			for (int I = wave; I < 4; I++) {
+				inv_scale(Li, I, wave - 1, inv_sum(S, Li, I, wave - 1));
+				wave_lds_order();
+			}
 	}
-	// off-diagonal blocks of inv(L): Li_IJ = -Li_II * sum_{K=J}^{I-1} L_IK Li_KJ
-	for (int d = 1; d < 4; d++) {
-		if (wave < 4 - d) {
-			const int J = wave, I = J + d;
-			V Tb = zero4<T>();
-			for (int K = J; K < I; K++)
-				Tb = mm16_nn(&S[16 * I + 16 * K * LD], &Li[16 * K + 16 * J * LD], Tb);
-			const V X = mm16_nreg(&Li[16 * I + 16 * I * LD], Tb, zero4<T>());
-			st16(&Li[16 * I + 16 * J * LD], X, T(-1));
-		}
-		__syncthreads();
-	}
-	if (FACTOR)
-		for (int idx = tid; idx < 64 * 64; idx += 256) {
-			const int i = idx & 63, j = idx >> 6;
+	__syncthreads();
+	// LDS reads of a thread ahead of its stores, as for the loads
+	T o[16];
+	if (FACTOR) {
+#pragma unroll
+		for (int q = 0; q < 16; q++)
+			o[q] = S[((tid + 256 * q) & 63) + ((tid + 256 * q) >> 6) * LD];
+#pragma unroll
+		for (int q = 0; q < 16; q++) {
+			const int i = (tid + 256 * q) & 63, j = (tid + 256 * q) >> 6;
 			if (i < w && j < w && i >= j)
-				D[i + (long)j * ldd] = S[i + j * LD];
+				D[i + (long)j * ldd] = o[q];
 		}
-	for (int idx = tid; idx < 64 * 64; idx += 256) {
-		const int i = idx & 63, j = idx >> 6;
-		Dinv[i + j * 64] = Li[i + j * LD];
 	}
+#pragma unroll
+	for (int q = 0; q < 16; q++)
+		o[q] = Li[((tid + 256 * q) & 63) + ((tid + 256 * q) >> 6) * LD];
+#pragma unroll
+	for (int q = 0; q < 16; q++)
+		Dinv[tid + 256 * q] = o[q];
 	__syncthreads();
 	return bad;
 }
