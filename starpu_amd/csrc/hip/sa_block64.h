@@ -202,10 +202,11 @@ __device__ __forceinline__ float quot_nr(float x, float d, float y)
 // one pivot d to the next is kept short: the columns to the right take
 // x_j -= (x_k / d) x_jk with the unscaled multipliers x_jk, which are
 // broadcast while the quotient is formed; the column itself is scaled by
-// d^{-1/2} off that chain.  The broadcasts are v_readlane: the row-broadcast
-// DPP form reaches only the lanes of one 16-lane row.
-template <typename T>
-__device__ __forceinline__ int potrf16_regs(T (&x)[16])
+// d^{-1/2} off that chain and handed to done(k, column).  The broadcasts are
+// v_readlane: the row-broadcast DPP form reaches only the lanes of one
+// 16-lane row.
+template <typename T, typename F>
+__device__ __forceinline__ int potrf16_regs(T (&x)[16], F done)
 {
 	unsigned long long bad = 0;
 #pragma unroll
@@ -227,38 +228,70 @@ __device__ __forceinline__ int potrf16_regs(T (&x)[16])
 		for (int j = k + 1; j < 16; j++)
 			x[j] -= z * m[j];
 		x[k] *= rsqrt_nr(d);
+		done(k, x[k]);
 	}
 	return __ffsll((long long)bad);
 }
 
+// LDS written by other lanes of the same wave is read next: keep the order.
+__device__ __forceinline__ void wave_lds_order()
+{
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Inverse of the factored 16x16 lower diagonal block J of S into the same
-// block of Li (zeros above its diagonal), by one wave: lane c (mod 16) takes
-// column c.  One division per lane, all lanes at once, then the columns of L
-// from left to right: y_q = s_q / L(q,q), s_i -= L(i,q) y_q for i > q, whose
-// only chain is one product and one multiply-add per column; L(i,q) is read
-// from LDS as a broadcast, off that chain.  The block may just have been
-// factored or loaded: the inverse has the same bits.
+// block of Li (zeros above its diagonal), by one wave.  The two 8x8 diagonal
+// halves first, lane c (mod 16) taking column c of the one it falls in: one
+// division per lane, all lanes at once, then the columns of L from left to
+// right, y_q = s_q / L(q,q), s_i -= L(i,q) y_q for i > q (L from LDS, each
+// half's element a broadcast).  Then the block below by two 16x16x16 MFMA
+// products with everything but the needed quarter zero: -C^{-1} (B A^{-1}).
+// Half the chain and a quarter of the multiply-adds of sixteen columns in
+// one.  The block may just have been factored or loaded: the inverse has the
+// same bits.
 template <typename T>
 __device__ __forceinline__ void inv16(const T *S, int J, T *Li)
 {
-	const int lane = threadIdx.x & 63, c = lane & 15;
+	typedef typename V4<T>::type V;
+	const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, c = r & 7, h = r & 8;
 	const T *B = S + 16 * J + 16 * J * LD;
-	const T rd = T(1) / B[c + c * LD];
-	T y[16];
+	const T *H = B + h + h * LD;
+	T *I = Li + 16 * J + 16 * J * LD;
+	const T rd = T(1) / H[c + c * LD];
+	T y[8];
 #pragma unroll
-	for (int i = 0; i < 16; i++)
+	for (int i = 0; i < 8; i++)
 		y[i] = (c == i) ? T(1) : T(0);
 #pragma unroll
-	for (int q = 0; q < 16; q++) {
-		y[q] *= bcast(rd, q);
+	for (int q = 0; q < 8; q++) {
+		const T lo = bcast(rd, q), hi = bcast(rd, q + 8);
+		y[q] *= h ? hi : lo;
 #pragma unroll
-		for (int i = q + 1; i < 16; i++)
-			y[i] -= B[i + q * LD] * y[q];
+		for (int i = q + 1; i < 8; i++)
+			y[i] -= H[i + q * LD] * y[q];
 	}
+	// column r of the block: its half's rows, zero in the other half's
 	if (lane < 16)
 #pragma unroll
-		for (int i = 0; i < 16; i++)
-			Li[(16 * J + i) + (16 * J + c) * LD] = y[i];
+		for (int i = 0; i < 8; i++) {
+			I[i + r * LD] = h ? T(0) : y[i];
+			I[8 + i + r * LD] = h ? y[i] : T(0);
+		}
+	wave_lds_order();
+	V t = zero4<T>();
+#pragma unroll
+	for (int s = 0; s < 4; s++) {
+		const int k = 4 * s + g;
+		const T b = B[r + k * LD];
+		t = sa_mfma(r >= 8 && k < 8 ? b : T(0), I[k + r * LD], t);
+	}
+	const V x = mm16_nreg(I, t, zero4<T>());
+#pragma unroll
+	for (int q = 0; q < 4; q++)
+		if (drow<T>(q, g) >= 8 && r < 8)
+			I[drow<T>(q, g) + r * LD] = -x[q];
 }
 
 // sum_{K=J}^{I-1} L_IK Li_KJ, the product that block (I, J) of the inverse
@@ -278,34 +311,14 @@ __device__ __forceinline__ void inv_scale(T *Li, int I, int J, typename V4<T>::t
 	st16(&Li[16 * I + 16 * J * LD], mm16_nreg(&Li[16 * I + 16 * I * LD], t, zero4<T>()), T(-1));
 }
 
-// LDS written by other lanes of the same wave is read next: keep the order.
-__device__ __forceinline__ void wave_lds_order()
+// The w x w lower block D into S, identity past w, zeros above the diagonal;
+// Li zeroed.  All 16 loads of a thread are in flight before the first LDS
+// store (the block sits in L2; one round trip instead of sixteen).
+template <typename T>
+__device__ __forceinline__ void block_load64(int w, const T *__restrict__ D, long ldd, T *__restrict__ S,
+                                             T *__restrict__ Li)
 {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// FACTOR: Cholesky of the w x w (w <= 64) lower block D (ld ldd, in place)
-// and its inverse into Dinv (64 x 64, ld 64, identity past w).
-// !FACTOR: D is already factored; only the inverse is formed.
-// One 256-thread workgroup; S and Li are two LDS blocks of 64 * LD elements.
-// Bound: the 64 dependent columns.  Wave 0 runs them as four panels of 16
-// columns over all the rows below (potrf16_regs), and everything else
-// overlaps the next panel: the trailing blocks, the 16x16 inverses and the
-// columns of the inverse, one per wave.  Only the update of the next 16
-// columns stands between two panels.
-// Returns, in every thread of wave 0, the 1-based column of the first
-// non-positive pivot within the block (or 0); other threads return 0.
-// Ends with a workgroup barrier, so the caller may reuse S and Li.
-template <typename T, bool FACTOR>
-__device__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__restrict__ Dinv, T *__restrict__ S,
-                                   T *__restrict__ Li)
-{
-	typedef typename V4<T>::type V;
-	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-	// all 16 loads of a thread in flight before the first LDS store (the
-	// block sits in L2; one round trip instead of sixteen)
+	const int tid = threadIdx.x;
 	T v[16];
 #pragma unroll
 	for (int q = 0; q < 16; q++) {
@@ -321,35 +334,53 @@ __device__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__rest
 		Li[i + j * LD] = T(0);
 	}
 	__syncthreads();
+}
 
+// FACTOR: Cholesky of the lower block in S, in place, and its inverse into
+// the lower part of Li.  !FACTOR: S holds the factor already; only the
+// inverse is formed, with the same bits.  One 256-thread workgroup; S and Li
+// are two LDS blocks of 64 * LD elements, Li's blocks of 16 above the
+// diagonal zero on entry (they are not written); S above its diagonal is
+// neither used nor kept.  Returns, in every thread of wave 0, the 1-based
+// column of the first non-positive pivot within the block (or 0); other
+// threads return 0.  Ends with a workgroup barrier.
+// Bound: the 64 dependent columns.  Wave 0 runs them as four panels of 16
+// columns over all the rows below (potrf16_regs), and everything else
+// overlaps the next panel: the trailing blocks, the 16x16 inverses and the
+// columns of the inverse, one per wave.  Only the update of the next 16
+// columns stands between two panels.
+template <typename T, bool FACTOR>
+__device__ __forceinline__ int block_core64(T *__restrict__ S, T *__restrict__ Li)
+{
+	typedef typename V4<T>::type V;
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	int bad = 0;
 	if (FACTOR) {
 		// wave q = 1..3 keeps the sum of the next block of its inverse column
 		V t = zero4<T>();
 		const int Jc = wave - 1;
+		// not unrolled: one copy of the panel code, 16 columns of it, stays in
+		// the instruction cache
 #pragma unroll
 		for (int J = 0; J < 4; J++) {
 			if (wave == 0) {
+				// lanes past the block take the padding row 64 of each column, so
+				// that no branch breaks up the column loop
+				const int row = 16 * J + lane < 64 ? 16 * J + lane : 64;
+				T *P = S + row + 16 * J * LD;
 				T x[16];
-				const int row = 16 * J + lane;
 #pragma unroll
 				for (int c = 0; c < 16; c++)
-					x[c] = row < 64 ? S[row + (16 * J + c) * LD] : T(0);
-				const int b = potrf16_regs(x);
+					x[c] = P[c * LD];
+				// the diagonal block's upper half, which nothing reads, receives
+				// what the elimination leaves there
+				const int b = potrf16_regs(x, [&](int c, T v) { P[c * LD] = v; });
 				if (b && !bad)
 					bad = 16 * J + b;
-				// the diagonal block's upper half, which nothing reads, holds
-				// what the elimination left there
-				if (row < 64)
-#pragma unroll
-					for (int c = 0; c < 16; c++)
-						S[row + (16 * J + c) * LD] = x[c];
 			} else if (J > 0) {
 				// trailing blocks right of column block J, by column block J - 1
 				int p = 0;
-#pragma unroll
 				for (int K = J + 1; K < 4; K++)
-#pragma unroll
 					for (int I = K; I < 4; I++, p++)
 						if (p % 3 == wave - 1) {
 							V acc = ld16(&S[16 * I + 16 * K * LD]);
@@ -399,25 +430,56 @@ __device__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__rest
 			}
 	}
 	__syncthreads();
-	// LDS reads of a thread ahead of its stores, as for the loads
+	return bad;
+}
+
+// Element (i, j) and its index in an LDS block for item q of 16 of a thread.
+__device__ __forceinline__ int b64_i(int q) { return (threadIdx.x + 256 * q) & 63; }
+__device__ __forceinline__ int b64_j(int q) { return (threadIdx.x + 256 * q) >> 6; }
+
+// Lower part of S into D (w x w), LDS reads of a thread ahead of its stores.
+template <typename T>
+__device__ __forceinline__ void store_lower64(int w, const T *__restrict__ S, T *__restrict__ D, long ldd)
+{
 	T o[16];
-	if (FACTOR) {
 #pragma unroll
-		for (int q = 0; q < 16; q++)
-			o[q] = S[((tid + 256 * q) & 63) + ((tid + 256 * q) >> 6) * LD];
+	for (int q = 0; q < 16; q++)
+		o[q] = S[b64_i(q) + b64_j(q) * LD];
 #pragma unroll
-		for (int q = 0; q < 16; q++) {
-			const int i = (tid + 256 * q) & 63, j = (tid + 256 * q) >> 6;
-			if (i < w && j < w && i >= j)
-				D[i + (long)j * ldd] = o[q];
-		}
+	for (int q = 0; q < 16; q++) {
+		const int i = b64_i(q), j = b64_j(q);
+		if (i < w && j < w && i >= j)
+			D[i + (long)j * ldd] = o[q];
 	}
+}
+
+// Li into Dinv (64 x 64, ld 64).
+template <typename T>
+__device__ __forceinline__ void store_inv64(const T *__restrict__ Li, T *__restrict__ Dinv)
+{
+	T o[16];
 #pragma unroll
 	for (int q = 0; q < 16; q++)
-		o[q] = Li[((tid + 256 * q) & 63) + ((tid + 256 * q) >> 6) * LD];
+		o[q] = Li[b64_i(q) + b64_j(q) * LD];
 #pragma unroll
 	for (int q = 0; q < 16; q++)
-		Dinv[tid + 256 * q] = o[q];
+		Dinv[threadIdx.x + 256 * q] = o[q];
+}
+
+// FACTOR: Cholesky of the w x w (w <= 64) lower block D (ld ldd, in place)
+// and its inverse into Dinv (64 x 64, ld 64, identity past w).
+// !FACTOR: D is already factored; only the inverse is formed.
+// One 256-thread workgroup; S, Li and the result as block_core64.  Ends with
+// a workgroup barrier, so the caller may reuse S and Li.
+template <typename T, bool FACTOR>
+__device__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__restrict__ Dinv, T *__restrict__ S,
+                                   T *__restrict__ Li)
+{
+	block_load64<T>(w, D, ldd, S, Li);
+	const int bad = block_core64<T, FACTOR>(S, Li);
+	if (FACTOR)
+		store_lower64<T>(w, S, D, ldd);
+	store_inv64<T>(Li, Dinv);
 	__syncthreads();
 	return bad;
 }

@@ -11,41 +11,62 @@
 // counters in device memory instead.
 //
 // Work is split into items on 64x64 blocks (block b covers rows and columns
-// 64b .. 64b+w_b-1 of the tile).  The factorisation:
-//   D(j)      factor and invert the diagonal block (j, j)        (LDS, MFMA)
-//   P(i,j)    L(i,j) = A(i,j) inv(L(j,j))^T                          (MFMA)
-//   U(i,l,j)  A(i,l) -= L(i,j) L(l,j)^T, j < l <= i (lower part if i = l)
-// and, when the inverse is asked for, W = L^-T (upper) block by block,
-// W(j,i) = -(sum_{t=j}^{i-1} W(j,t) L(i,t)^T) inv(L(i,i))^T, W(j,j) =
-// inv(L(j,j))^T:
-//   WD(t)     W(t,t) = inv(L(t,t))^T, the inverse D(t) formed
-//   WX(j,i)   the sum over t in registers, taking each product as soon as
-//             W(j,t) and L(i,t) are final, then the scaling by
-//             inv(L(i,i))^T (MFMA); one store and one publication per block
+// 64b .. 64b+w_b-1 of the tile), left-looking: an item owns one block, sums
+// its products over all the columns to its left in registers and touches
+// the block in memory once.  The factorisation:
+//   chain(j)  by workgroup 0, which keeps the blocks of its step in LDS:
+//             D(j) factors and inverts the diagonal block, L(j+1,j) =
+//             A(j+1,j) inv(L(j,j))^T, and the last update of the next
+//             diagonal block, A(j+1,j+1) -= L(j+1,j) L(j+1,j)^T, stays in LDS
+//   S(j)      A(j+1,j) -= sum_{t<j} L(j+1,t) L(j,t)^T            (MFMA)
+//   G(j)      A(j+1,j+1) -= sum_{t<j} L(j+1,t) L(j+1,t)^T        (MFMA)
+//   P(i,j)    L(i,j) = (A(i,j) - sum_{t<j} L(i,t) L(j,t)^T) inv(L(j,j))^T
+//             for i > j + 1                                      (MFMA)
+// S and G prepare what the chain takes at step j; the product with t = j - 1
+// of S(j) is the only work that lies between two steps of the chain, and it
+// runs beside D(j).  When the inverse is asked for, W = L^-T (upper) block by
+// block, W(j,j) = inv(L(j,j))^T,
+// W(j,i) = -(sum_{t=j}^{i-1} W(j,t) L(i,t)^T) inv(L(i,i))^T:
+//   WD(t)     W(t,t), from the inverse D(t) formed
+//   WX(j,i)   W(j,i), the sum in registers, one store
 // with Linv = L^-1 = W^T written beside W by WD and WX when asked for.
 // These are the inverse's flops (n^3/3) on the same matrix cores, overlapped
 // with the factorisation's critical chain instead of following it.
 //
 // Ordering and progress.  Every item depends only on items that come earlier
-// in one fixed global order: step by step, the critical chain D(j), P(j+1,j),
-// U(j+1,j+1,j), then the other factor items of step j, then the inverse
-// items of block column j - 1, WD(j-1) and WX(t, j-1) for t < j-1 (one step
-// late, so that the factor items the chain waits for come first).  Workgroup 0 runs the critical chain; the other
-// workgroups take the remaining items in that order from a ticket counter.
-// Each workgroup processes its items in increasing order, so the lowest
-// unfinished item always has all its inputs ready and a running workgroup
-// holds it: the grid always drains.  Block (i, l) of A carries a counter:
-// the number of updates applied, then +1 when the block is final; block
-// (j, i) of W is raised to 1 once final.  The updates of a block are
-// applied in step order, so the result does not depend on timing.  Inverting an already factored
-// tile (sa_dtrtri_tile) runs the same inverse items after D items that only
+// in one fixed global order: step by step, chain(j), S(j), G(j), P(i,j) from
+// i = j + 2 on, then the inverse items of block column j - 1, WD(j-1) and
+// WX(t, j-1) for t < j-1 (one step late, so that the factor items the chain
+// waits for come first).  Within a step chain(j) follows S(j) and G(j), which
+// need no more of step j than nothing: their inputs are of steps before it.
+// Workgroup 0 runs the chain; the other workgroups take the remaining items
+// in that order from a ticket counter.  Each workgroup processes its items in
+// increasing order, so the lowest unfinished item always has all its inputs
+// ready and a running workgroup holds it: the grid always drains.  The blocks
+// of a row of L (and of W) become final from left to right, each after the
+// one before it, so one counter per row tells how many are: an item reads
+// two counters and then runs through every product that is ready without
+// another look.  The products of a block are added in the order of t, so the
+// result does not depend on timing.  Inverting an already factored tile
+// (sa_dtrtri_tile) runs the same inverse items after D items that only
 // invert, so a solve on a resident factor multiplies by the same bits.
+//
+// Bound: the chain, 17.7 us a step alone on the chip (8.5 the block, 3.3 the
+// stores, the look at what is prepared and its loads, 1.9 the panel product,
+// 1.3 its publication, 2.4 the diagonal update), from about 31 bulk
+// workgroups on up to n = 1024, and the bulk beyond: a 1024 tile with both
+// inverses takes 349 us with 31 workgroups, a 2048 tile 1580 with 31, 1020
+// with 63 and 785 with 127.  One item per block and update step (right-looking),
+// each block read and written at every step and the chain's blocks handed
+// on through memory, took 43 us a step and 1357, 1056 and 907 us for a 1024
+// tile with 31, 63 and 127.
 //
 // Every wait is bounded: a counter that does not reach its value within
 // seconds (which cannot happen unless the order above is broken) raises
-// an abort flag that ends every workgroup's loop, and the factorisation then
-// reports info = -1, so a fault of the ordering shows as an error, not as a
-// hung device.
+// an abort flag, after which no wait waits any more: every workgroup runs
+// through its items on whatever memory holds (in bounds all the same), the
+// grid drains and the factorisation reports info = -1, so a fault of the
+// ordering shows as an error, not as a hung device.
 //
 // Visibility across workgroups (possibly on different XCDs, each with its own
 // L2) uses agent-scope release fences before a counter is raised and an
@@ -75,6 +96,12 @@ int max_bulk()
 	return v;
 }
 
+// The counters, each on a 64-byte line of its own: rows of L, then
+// "A(i,i) / A(i+1,i) prepared" and "D(i) done" flags, rows of W, the ticket
+// and the abort flag.
+constexpr int FLAG_STRIDE = 16;       // unsigned per line
+constexpr int flag_words(int nb) { return (5 * nb + 2) * FLAG_STRIDE; }
+
 struct PfArgs {
 	int n, nb, nbulk;
 	int factor;         // 1: factor A in place; 0: A holds the factor already
@@ -87,67 +114,51 @@ struct PfArgs {
 	double *Linv;
 	long ldi;
 	double *Dinv;       // nb blocks of 64x64 (ld 64)
-	unsigned *fa;       // counters of the blocks of A: index i + nb * l
-	unsigned *ticket;   // next item of the bulk order to hand out
-	unsigned *abort;    // raised by a wait that ran out
-	unsigned *fw;       // counters of the blocks of W: index j + nb * i
+	unsigned *flags;
 	int *info;
+	__device__ unsigned *rowl(int i) const { return flags + FLAG_STRIDE * i; }          // L(i,t) final for t < value
+	__device__ unsigned *diag(int i) const { return flags + FLAG_STRIDE * (nb + i); }   // A(i,i) but for t = i - 1
+	__device__ unsigned *sub(int i) const { return flags + FLAG_STRIDE * (2 * nb + i); } // A(i+1,i), all t < i
+	__device__ unsigned *dfin(int i) const { return flags + FLAG_STRIDE * (3 * nb + i); }
+	__device__ unsigned *roww(int j) const { return flags + FLAG_STRIDE * (4 * nb + j); } // W(j,t) final for t < value
+	__device__ unsigned *ticket() const { return flags + FLAG_STRIDE * (5 * nb); }
+	__device__ unsigned *abortf() const { return flags + FLAG_STRIDE * (5 * nb + 1); }
 };
 
 __device__ __forceinline__ int bw(const PfArgs &p, int b) { return (p.n - 64 * b) < 64 ? (p.n - 64 * b) : 64; }
 
-// A wait gives up after SPIN_LIMIT polls.  Each poll is two device-coherent
-// loads of about a microsecond and a short sleep, so 2^22 polls are several
-// seconds: far beyond any wait of a correct schedule (an item takes tens of
-// microseconds).
+__device__ __forceinline__ unsigned flag_read(const unsigned *f)
+{
+	return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A wait gives up after SPIN_LIMIT polls.  Each poll is two or three
+// device-coherent loads of about a microsecond and a short sleep, so 2^22
+// polls are several seconds: far beyond any wait of a correct schedule (an
+// item takes tens of microseconds).
 constexpr unsigned SPIN_LIMIT = 1u << 22;
 
-__device__ __forceinline__ bool spin(const unsigned *f, unsigned v, unsigned *abortf)
+// One wave waits until both counters have reached v (or the run is
+// abandoned) and then sees the data published before they were raised.
+// Returns the smaller counter, at least v.
+__device__ __forceinline__ int await(const PfArgs &p, const unsigned *f1, const unsigned *f2, int v)
 {
 	unsigned it = 0;
-	while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) {
-		if (__hip_atomic_load(abortf, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-			return false;
-		if (++it > SPIN_LIMIT) {
-			__hip_atomic_store(abortf, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			return false;
+	int m;
+	for (;;) {
+		const int a = (int)flag_read(f1), b = (int)flag_read(f2);
+		m = __builtin_amdgcn_readfirstlane(a < b ? a : b);
+		if (m >= v)
+			break;
+		if (__builtin_amdgcn_readfirstlane((int)flag_read(p.abortf())) || ++it > SPIN_LIMIT) {
+			__hip_atomic_store(p.abortf(), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			m = v;
+			break;
 		}
 		__builtin_amdgcn_s_sleep(1);
 	}
-	return true;
-}
-
-// Thread 0 waits until each given counter reaches its value; the whole
-// workgroup then sees the data published before those counters were raised.
-// False (in every thread) if the wait was abandoned.
-__device__ __forceinline__ bool wait_for(const PfArgs &p, const unsigned *f1, unsigned v1,
-                                         const unsigned *f2 = nullptr, unsigned v2 = 0,
-                                         const unsigned *f3 = nullptr, unsigned v3 = 0)
-{
-	__shared__ int s_ok;
-	if (threadIdx.x == 0) {
-		bool ok = !f1 || spin(f1, v1, p.abort);
-		ok = ok && (!f2 || spin(f2, v2, p.abort));
-		ok = ok && (!f3 || spin(f3, v3, p.abort));
-		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-		s_ok = ok ? 1 : 0;
-	}
-	__syncthreads();
-	const bool ok = s_ok != 0;
-	__syncthreads();
-	return ok;
-}
-
-// The abort flag as the whole workgroup sees it (one read, broadcast).
-__device__ __forceinline__ bool aborted(const PfArgs &p)
-{
-	__shared__ int s_ab;
-	if (threadIdx.x == 0)
-		s_ab = __hip_atomic_load(p.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? 1 : 0;
-	__syncthreads();
-	const bool a = s_ab != 0;
-	__syncthreads();
-	return a;
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+	return m;
 }
 
 // Every thread's stores become visible at agent scope, then the counter is
@@ -163,56 +174,133 @@ __device__ __forceinline__ void publish(unsigned *f, unsigned v)
 		__hip_atomic_store(f, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// acc += Pr Pc^T over k < wk for the wave's 32x32 quadrant (rows i0.., cols
-// j0.., i0 = 32 (wave & 1), j0 = 32 (wave >> 1)) of a wr x wc block; Pr
-// (wr x wk, ld ldr), Pc (wc x wk, ld ldpc).  The MFMA computes the transposed
-// product so a lane's results are consecutive rows: acc[bj][bi][q] =
-// (Pr Pc^T)(i0 + 16 bi + r, j0 + 16 bj + 4q + g).  Operand loads in two
-// batches of half the k range: the blocks sit in L2 and the item is
-// latency-bound.
-__device__ __forceinline__ void acc_nt(int wr, int wc, int wk, const double *__restrict__ Pr, long ldr,
-                                       const double *__restrict__ Pc, long ldpc, sa_d4 (&acc)[2][2])
+// acc += Pr Pc^T over the columns 64 t0 .. 64 t1 - 1 of two block rows, for
+// the wave's 32x32 quadrant (rows i0 = 32 (wave & 1).., columns j0 = 32
+// (wave >> 1)..).  Pr and Pc are the lanes' addresses of column 0 in the two
+// block rows: rows r and r + 16 of the quadrant's half, columns k = 4s + g.
+// The MFMA computes the transposed product so a lane's results are
+// consecutive rows: acc[bj][bi][q] = (Pr Pc^T)(i0 + 16 bi + r,
+// j0 + 16 bj + 4q + g).  Blocks t of the two rows are ready for t below both
+// counters.  Operands come in stages of 32 columns, one stage ahead of the
+// MFMAs; while a block's first half is multiplied the counters are read
+// again, so that a run goes on without a pause when more has become ready.
+struct Operand {
+	const double *p[2];     // the lane's two rows, column g
+	long ld;
+};
+
+__device__ __forceinline__ Operand operand(const double *X, long ld, int row0, int last)
 {
-	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
-	double xa[2][8], xb[2][8];
+	const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+	Operand o;
 #pragma unroll
-	for (int h = 0; h < 2; h++) {
+	for (int b = 0; b < 2; b++) {
+		const int row = row0 + 16 * b + r;
+		o.p[b] = X + (row < last ? row : last) + g * ld;
+	}
+	o.ld = ld;
+	return o;
+}
+
+__device__ __forceinline__ void load_half(const Operand &o, int k, double (&x)[2][8])
+{
 #pragma unroll
-		for (int s = 0; s < 8; s++) {
-			const int k = 4 * (8 * h + s) + g;
-			const bool kin = k < wk;
-			const long kr = (long)(kin ? k : 0) * ldr, kc = (long)(kin ? k : 0) * ldpc;
+	for (int s = 0; s < 8; s++)
 #pragma unroll
-			for (int b = 0; b < 2; b++) {
-				const int rj = j0 + 16 * b + r, ri = i0 + 16 * b + r;
-				const double va = Pc[(rj < wc ? rj : 0) + kc];
-				const double vb = Pr[(ri < wr ? ri : 0) + kr];
-				xa[b][s] = (kin && rj < wc) ? va : 0.0;
-				xb[b][s] = (kin && ri < wr) ? vb : 0.0;
+		for (int b = 0; b < 2; b++)
+			x[b][s] = o.p[b][(long)(k + 4 * s) * o.ld];
+}
+
+__device__ __forceinline__ void mul_half(const double (&xr)[2][8], const double (&xc)[2][8], sa_d4 (&acc)[2][2])
+{
+#pragma unroll
+	for (int s = 0; s < 8; s++)
+#pragma unroll
+		for (int bj = 0; bj < 2; bj++)
+#pragma unroll
+			for (int bi = 0; bi < 2; bi++)
+				acc[bj][bi] = sa_mfma(xc[bj][s], xr[bi][s], acc[bj][bi]);
+}
+
+__device__ __forceinline__ void accumulate(const PfArgs &p, const Operand &Pr, const Operand &Pc,
+                                           const unsigned *fr, const unsigned *fc, int t0, int t1,
+                                           sa_d4 (&acc)[2][2])
+{
+	double r0[2][8], c0[2][8], r1[2][8], c1[2][8];
+#pragma unroll
+	for (int a = 0; a < 2; a++)
+#pragma unroll
+		for (int b = 0; b < 2; b++)
+			acc[a][b] = sa_d4{0.0, 0.0, 0.0, 0.0};
+	int ready = t0;
+	bool staged = false;            // the first half of block t is in r0, c0
+	for (int t = t0; t < t1; t++) {
+		if (!staged) {
+			if (ready <= t)
+				ready = await(p, fr, fc, t + 1);
+			load_half(Pr, 64 * t, r0);
+			load_half(Pc, 64 * t, c0);
+		}
+		load_half(Pr, 64 * t + 32, r1);
+		load_half(Pc, 64 * t + 32, c1);
+		unsigned fa = 0, fb = 0;
+		const bool look = ready <= t + 1 && t + 1 < t1;
+		if (look) {
+			fa = flag_read(fr);
+			fb = flag_read(fc);
+		}
+		mul_half(r0, c0, acc);
+		if (look) {
+			const int m = __builtin_amdgcn_readfirstlane((int)(fa < fb ? fa : fb));
+			if (m > ready) {
+				__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+				ready = m;
 			}
 		}
-#pragma unroll
-		for (int s = 0; s < 8; s++)
-#pragma unroll
-			for (int bj = 0; bj < 2; bj++)
-#pragma unroll
-				for (int bi = 0; bi < 2; bi++)
-					acc[bj][bi] = sa_mfma(xa[bj][s], xb[bi][s], acc[bj][bi]);
+		staged = t + 1 < t1 && ready > t + 1;
+		if (staged) {
+			load_half(Pr, 64 * t + 64, r0);
+			load_half(Pc, 64 * t + 64, c0);
+		}
+		mul_half(r1, c1, acc);
 	}
 }
 
-// C (wr x wc, ld ldc) -= Pr Pc^T over k < wk; lower part only if LOWER.
-// Each wave a 32x32 quadrant (acc_nt); the quadrant of C is loaded with
-// the operands and written once.
-__device__ __forceinline__ void upd_nt(int wr, int wc, int wk, const double *__restrict__ Pr, long ldr,
-                                       const double *__restrict__ Pc, long ldpc, double *__restrict__ C, long ldc,
-                                       bool lower)
+// X = T inv^T for the wave's 16 rows 16 wave ..: T (64x64) in LDS, inv a
+// lower 64x64 block with leading dimension ldd (its zeros above the diagonal
+// are not multiplied).  x[cb][q] = X(16 wave + r, 16 cb + 4q + g).
+__device__ __forceinline__ void apply_inv(const double *T, const double *Dj, long ldd, sa_d4 (&x)[4])
+{
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+	double dv[40];
+#pragma unroll
+	for (int cb = 0, q = 0; cb < 4; cb++)
+#pragma unroll
+		for (int s = 0; s < 4 * (cb + 1); s++, q++)
+			dv[q] = Dj[(16 * cb + r) + (4 * s + g) * ldd];
+#pragma unroll
+	for (int cb = 0; cb < 4; cb++)
+		x[cb] = sa_d4{0.0, 0.0, 0.0, 0.0};
+	// k outermost: the four column blocks are independent accumulators
+#pragma unroll
+	for (int s = 0; s < 16; s++) {
+		const double t = T[(16 * wave + r) + (4 * s + g) * LD];
+#pragma unroll
+		for (int cb = 0; cb < 4; cb++)
+			if (s < 4 * (cb + 1))
+				x[cb] = sa_mfma(dv[2 * cb * (cb + 1) + s], t, x[cb]);
+	}
+}
+
+// ---- factorisation items ---------------------------------------------------
+
+// S(j) (l = j) and G(j) (l = j + 1): A(j+1,l) -= sum_{t<j} L(j+1,t) L(l,t)^T.
+__device__ __noinline__ void item_prepare(const PfArgs &p, int j, int l)
 {
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
-	if (lower && j0 > i0 + 31)
-		return;
+	const int i = j + 1, wr = bw(p, i), wc = bw(p, l);
+	double *C = p.A + 64 * i + 64L * l * p.lda;
 	double cv[2][4][2];
 #pragma unroll
 	for (int bj = 0; bj < 2; bj++)
@@ -221,15 +309,11 @@ __device__ __forceinline__ void upd_nt(int wr, int wc, int wk, const double *__r
 #pragma unroll
 			for (int bi = 0; bi < 2; bi++) {
 				const int ic = i0 + 16 * bi + r, jc = j0 + 16 * bj + 4 * q + g;
-				cv[bj][q][bi] = C[(ic < wr ? ic : 0) + (long)(jc < wc ? jc : 0) * ldc];
+				cv[bj][q][bi] = C[(ic < wr ? ic : 0) + (long)(jc < wc ? jc : 0) * p.lda];
 			}
 	sa_d4 acc[2][2];
-#pragma unroll
-	for (int a = 0; a < 2; a++)
-#pragma unroll
-		for (int b = 0; b < 2; b++)
-			acc[a][b] = sa_d4{0.0, 0.0, 0.0, 0.0};
-	acc_nt(wr, wc, wk, Pr, ldr, Pc, ldpc, acc);
+	accumulate(p, operand(p.A, p.lda, 64 * i + i0, p.n - 1), operand(p.A, p.lda, 64 * l + j0, p.n - 1), p.rowl(i),
+	           p.rowl(l), 0, j, acc);
 #pragma unroll
 	for (int bj = 0; bj < 2; bj++)
 #pragma unroll
@@ -237,58 +321,67 @@ __device__ __forceinline__ void upd_nt(int wr, int wc, int wk, const double *__r
 #pragma unroll
 			for (int bi = 0; bi < 2; bi++) {
 				const int ic = i0 + 16 * bi + r, jc = j0 + 16 * bj + 4 * q + g;
-				if (ic < wr && jc < wc && (!lower || ic >= jc))
-					C[ic + (long)jc * ldc] = cv[bj][q][bi] - acc[bj][bi][q];
+				if (ic < wr && jc < wc && (l != i || ic >= jc))
+					C[ic + (long)jc * p.lda] = cv[bj][q][bi] - acc[bj][bi][q];
 			}
+	publish(l == i ? p.diag(i) : p.sub(j), 1u);
 }
 
-// ---- factorisation items ---------------------------------------------------
-
-// The chain applies the last update of block (j, j) itself just before
-// D(j) (chain_U), so D(j) has no wait of its own.  Without FACTOR (the tile
-// is factored already) D(j) forms the inverse of the diagonal block only.
-template <bool FACTOR>
-__device__ __noinline__ void item_D(const PfArgs &p, int j, double *S, double *Li, int &first_bad)
+// T = C - sum in LDS, for P and (C = 0) WX; columns from wc on are zero.
+__device__ __forceinline__ void stage_block(const double (&cv)[2][4][2], const sa_d4 (&acc)[2][2], int wc, double *T)
 {
-	const int wj = bw(p, j);
-	const int bad = block_potrf_inv64<FACTOR>(wj, p.A + 64 * j + 64L * j * p.lda, p.lda, p.Dinv + 4096L * j, S, Li);
-	if (FACTOR && threadIdx.x == 0 && bad && bad <= wj && first_bad == 0)
-		first_bad = 64 * j + bad;
-	publish(&p.fa[j + p.nb * j], (unsigned)j + 1);
-}
-
-__device__ __noinline__ void item_P(const PfArgs &p, int i, int j)
-{
-	if (!wait_for(p, &p.fa[j + p.nb * j], (unsigned)j + 1, &p.fa[i + p.nb * j], (unsigned)j))
-		return;
-	rows_apply_inv((threadIdx.x >> 6) * 16, bw(p, i), bw(p, j), p.Dinv + 4096L * j,
-	               p.A + 64 * i + 64L * j * p.lda, p.lda);
-	publish(&p.fa[i + p.nb * j], (unsigned)j + 1);
-}
-
-__device__ __noinline__ void item_U(const PfArgs &p, int i, int l, int j)
-{
-	if (!wait_for(p, &p.fa[i + p.nb * j], (unsigned)j + 1, &p.fa[l + p.nb * j], (unsigned)j + 1,
-	              &p.fa[i + p.nb * l], (unsigned)j))
-		return;
-	const long lda = p.lda;
-	upd_nt(bw(p, i), bw(p, l), bw(p, j), p.A + 64 * i + 64L * j * lda, lda, p.A + 64 * l + 64L * j * lda, lda,
-	       p.A + 64 * i + 64L * l * lda, lda, i == l);
-	publish(&p.fa[i + p.nb * l], (unsigned)j + 1);
-}
-
-// U(j+1,j+1,j) on the critical chain: after the bulk updates of steps < j
-// (counter >= j), and not published, since only D(j+1) on this workgroup
-// consumes it (the counter goes from j to j+2 when D(j+1) is done).
-__device__ __noinline__ bool chain_U(const PfArgs &p, int j)
-{
-	if (!wait_for(p, &p.fa[(j + 1) + p.nb * (j + 1)], (unsigned)j))
-		return false;
-	const long lda = p.lda;
-	upd_nt(bw(p, j + 1), bw(p, j + 1), bw(p, j), p.A + 64 * (j + 1) + 64L * j * lda, lda,
-	       p.A + 64 * (j + 1) + 64L * j * lda, lda, p.A + 64 * (j + 1) + 64L * (j + 1) * lda, lda, true);
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
+#pragma unroll
+	for (int bj = 0; bj < 2; bj++)
+#pragma unroll
+		for (int q = 0; q < 4; q++)
+#pragma unroll
+			for (int bi = 0; bi < 2; bi++) {
+				const int ic = i0 + 16 * bi + r, jc = j0 + 16 * bj + 4 * q + g;
+				T[ic + jc * LD] = jc < wc ? cv[bj][q][bi] - acc[bj][bi][q] : 0.0;
+			}
 	__syncthreads();
-	return true;
+}
+
+__device__ __noinline__ void item_P(const PfArgs &p, int i, int j, double *T)
+{
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
+	const int wr = bw(p, i);            // block column j < i is full
+	double *C = p.A + 64 * i + 64L * j * p.lda;
+	double cv[2][4][2];
+#pragma unroll
+	for (int bj = 0; bj < 2; bj++)
+#pragma unroll
+		for (int q = 0; q < 4; q++)
+#pragma unroll
+			for (int bi = 0; bi < 2; bi++) {
+				const int ic = i0 + 16 * bi + r, jc = j0 + 16 * bj + 4 * q + g;
+				cv[bj][q][bi] = C[(ic < wr ? ic : 0) + (long)jc * p.lda];
+			}
+	sa_d4 acc[2][2];
+	accumulate(p, operand(p.A, p.lda, 64 * i + i0, p.n - 1), operand(p.A, p.lda, 64 * j + j0, p.n - 1), p.rowl(i),
+	           p.rowl(j), 0, j, acc);
+	stage_block(cv, acc, 64, T);
+	await(p, p.dfin(j), p.dfin(j), 1);
+	sa_d4 x[4];
+	apply_inv(T, p.Dinv + 4096L * j, 64, x);
+	const int row = 16 * wave + r;
+	if (row < wr)
+#pragma unroll
+		for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+				C[row + (long)(16 * cb + 4 * q + g) * p.lda] = x[cb][q];
+	publish(p.rowl(i), (unsigned)j + 1);
+}
+
+// The inverse of diagonal block j of a tile that is factored already.
+__device__ __noinline__ void item_D(const PfArgs &p, int j, double *S, double *Li)
+{
+	block_potrf_inv64<false>(bw(p, j), p.A + 64 * j + 64L * j * p.lda, p.lda, p.Dinv + 4096L * j, S, Li);
+	publish(p.dfin(j), 1u);
 }
 
 // ---- inverse items ---------------------------------------------------------
@@ -297,191 +390,231 @@ __device__ __noinline__ bool chain_U(const PfArgs &p, int j)
 // inv(L(t,t)) (lower; zero above), from the block inverse D(t) formed.
 __device__ __noinline__ void item_WD(const PfArgs &p, int t)
 {
-	if (!wait_for(p, &p.fa[t + p.nb * t], (unsigned)t + 1))
-		return;
+	await(p, p.dfin(t), p.dfin(t), 1);
 	const int w = bw(p, t);
 	const double *D = p.Dinv + 4096L * t;
 	double *Wb = p.W + 64 * t + 64L * t * p.ldw;
-	for (int idx = threadIdx.x; idx < 4096; idx += 256) {
-		const int i = idx & 63, j = idx >> 6;
+	double u[16], v[16];
+#pragma unroll
+	for (int q = 0; q < 16; q++) {
+		const int i = b64_i(q), j = b64_j(q);
+		u[q] = D[j + 64 * i];
+		v[q] = D[i + 64 * j];
+	}
+#pragma unroll
+	for (int q = 0; q < 16; q++) {
+		const int i = b64_i(q), j = b64_j(q);
 		if (i < w && j < w) {
-			Wb[i + (long)j * p.ldw] = i <= j ? D[j + 64 * i] : 0.0;
+			Wb[i + (long)j * p.ldw] = i <= j ? u[q] : 0.0;
 			if (p.Linv)
-				p.Linv[(64 * t + i) + (64L * t + j) * p.ldi] = i >= j ? D[i + 64 * j] : 0.0;
+				p.Linv[(64 * t + i) + (64L * t + j) * p.ldi] = i >= j ? v[q] : 0.0;
 		}
 	}
-	publish(&p.fw[t + p.nb * t], 1u);
+	publish(p.roww(t), (unsigned)t + 1);
 }
 
-// W(j,i) for j < i: the sum of W(j,t) L(i,t)^T over t = j..i-1 in
-// registers, each product taken as soon as its two blocks are final, then
-// W(j,i) = -sum inv(L(i,i))^T in place, with Linv(i,j) = W(j,i)^T; the
-// mirrored blocks W(i,j) and Linv(j,i) are zero.
-__device__ __noinline__ void item_WX(const PfArgs &p, int j, int i)
+// W(j,i) for j < i: the sum of W(j,t) L(i,t)^T over t = j..i-1 in registers,
+// then W(j,i) = -sum inv(L(i,i))^T, with Linv(i,j) = W(j,i)^T; the mirrored
+// blocks W(i,j) and Linv(j,i) are zero.
+__device__ __noinline__ void item_WX(const PfArgs &p, int j, int i, double *T, double *X)
 {
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
-	const int wr = bw(p, j), wc = bw(p, i);
+	const int wc = bw(p, i);            // block row j < i is full
 	sa_d4 acc[2][2];
-#pragma unroll
-	for (int a = 0; a < 2; a++)
-#pragma unroll
-		for (int b = 0; b < 2; b++)
-			acc[a][b] = sa_d4{0.0, 0.0, 0.0, 0.0};
-	for (int t = j; t < i; t++) {
-		if (!wait_for(p, &p.fw[j + p.nb * t], 1u, &p.fa[i + p.nb * t], (unsigned)t + 1))
-			return;
-		acc_nt(wr, wc, bw(p, t), p.W + 64 * j + 64L * t * p.ldw, p.ldw, p.A + 64 * i + 64L * t * p.lda, p.lda,
-		       acc);
-	}
-	if (!wait_for(p, &p.fa[i + p.nb * i], (unsigned)i + 1))
-		return;
+	accumulate(p, operand(p.W, p.ldw, 64 * j + i0, p.n - 1), operand(p.A, p.lda, 64 * i + j0, p.n - 1), p.roww(j),
+	           p.rowl(i), j, i, acc);
+	const double zero[2][4][2] = {};
+	stage_block(zero, acc, wc, T);
+	await(p, p.dfin(i), p.dfin(i), 1);
+	sa_d4 x[4];
+	apply_inv(T, p.Dinv + 4096L * i, 64, x);
+	const int row = 16 * wave + r;
 	double *Wb = p.W + 64 * j + 64L * i * p.ldw;
 #pragma unroll
-	for (int bj = 0; bj < 2; bj++)
+	for (int cb = 0; cb < 4; cb++)
 #pragma unroll
-		for (int q = 0; q < 4; q++)
-#pragma unroll
-			for (int bi = 0; bi < 2; bi++) {
-				const int ic = i0 + 16 * bi + r, jc = j0 + 16 * bj + 4 * q + g;
-				if (ic < wr && jc < wc)
-					Wb[ic + (long)jc * p.ldw] = -acc[bj][bi][q];
-			}
-	// the block's rows, written by all four waves, are read back by each
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-	__syncthreads();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-	rows_apply_inv_t<double>(wave * 16, wr, wc, p.Dinv + 4096L * i, Wb, p.ldw,
-	                         p.Linv ? p.Linv + 64 * i + 64L * j * p.ldi : nullptr, p.ldi);
-	for (int idx = threadIdx.x; idx < 4096; idx += 256) {
-		const int a = idx & 63, c = idx >> 6;
-		if (a < wc && c < wr)
+		for (int q = 0; q < 4; q++) {
+			const int c = 16 * cb + 4 * q + g;
+			if (c < wc)
+				Wb[row + (long)c * p.ldw] = x[cb][q];
+			if (p.Linv)
+				X[c + row * LD] = x[cb][q];
+		}
+	publish(p.roww(j), (unsigned)i + 1);
+	for (int q = 0; q < 16; q++) {
+		const int a = b64_i(q), c = b64_j(q);
+		if (a < wc)
 			p.W[(64 * i + a) + (64L * j + c) * p.ldw] = 0.0;
-		if (p.Linv && a < wr && c < wc)
-			p.Linv[(64 * j + a) + (64L * i + c) * p.ldi] = 0.0;
-	}
-	publish(&p.fw[j + p.nb * i], 1u);
-}
-
-__device__ void run_chain(const PfArgs &p, double *S, double *Li)
-{
-	int first_bad = 0;
-	for (int j = 0; j < p.nb; j++) {
-		item_D<true>(p, j, S, Li, first_bad);
-		if (j + 1 < p.nb) {
-			item_P(p, j + 1, j);
-			if (!chain_U(p, j))
-				break;
+		if (p.Linv) {
+			if (a < wc)
+				p.Linv[(64 * i + a) + (64L * j + c) * p.ldi] = X[a + c * LD];
+			if (c < wc)
+				p.Linv[(64 * j + a) + (64L * i + c) * p.ldi] = 0.0;
 		}
 	}
-	if (aborted(p))
-		first_bad = -1;
+}
+
+// ---- the critical chain ----------------------------------------------------
+
+// Step j: S (LDS) holds A(j,j) with all its updates.  The block is factored
+// and inverted in LDS and its inverse published; L(j+1,j) is formed from the
+// prepared A(j+1,j) and the inverse in LDS, published, and kept in LDS for
+// the last update of A(j+1,j+1), which becomes the next S.
+__device__ void run_chain(const PfArgs &p, double *S, double *Li)
+{
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+	int first_bad = 0;
+	if (p.nb > 0)
+		block_load64<double>(bw(p, 0), p.A, p.lda, S, Li);
+	for (int j = 0; j < p.nb; j++) {
+		const int wj = bw(p, j);
+		const int bad = block_core64<double, true>(S, Li);
+		if (threadIdx.x == 0 && bad && bad <= wj && first_bad == 0)
+			first_bad = 64 * j + bad;
+		store_inv64<double>(Li, p.Dinv + 4096L * j);
+		store_lower64<double>(wj, S, p.A + 64 * j + 64L * j * p.lda, p.lda);
+		if (j + 1 == p.nb) {
+			publish(p.dfin(j), 1u);
+			break;
+		}
+		const int wn = bw(p, j + 1);
+		double *P = p.A + 64 * (j + 1) + 64L * j * p.lda, *C = p.A + 64 * (j + 1) + 64L * (j + 1) * p.lda;
+		// the wave's 16 rows of A(j+1,j), and its blocks of the lower half of
+		// A(j+1,j+1): 16x16 blocks 4u + wave of the ten, row by row
+		const int row = 16 * wave + r, rowc = row < wn ? row : wn - 1;
+		double t[16], cv[3][4];
+		auto load_next = [&] {
+#pragma unroll
+			for (int s = 0; s < 16; s++)
+				t[s] = P[rowc + (long)(4 * s + g) * p.lda];
+#pragma unroll
+			for (int u = 0; u < 3; u++) {
+				const int b = 4 * u + wave, I = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, K = b - I * (I + 1) / 2;
+#pragma unroll
+				for (int q = 0; q < 4; q++) {
+					const int ic = 16 * I + r, jc = 16 * K + 4 * q + g;
+					cv[u][q] = (b < 10 && ic < wn && jc < wn) ? C[ic + (long)jc * p.lda] : 0.0;
+				}
+			}
+		};
+		// they are mostly there by now: one look while the inverse is on its
+		// way to memory, and the loads in flight while it is published
+		const unsigned ra = flag_read(p.sub(j)), rb = flag_read(p.diag(j + 1));
+		const bool there = __builtin_amdgcn_readfirstlane((int)(ra & rb)) != 0;
+		if (there) {
+			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+			load_next();
+		}
+		publish(p.dfin(j), 1u);
+		if (!there) {
+			await(p, p.sub(j), p.diag(j + 1), 1);
+			load_next();
+		}
+		sa_d4 x[4];
+#pragma unroll
+		for (int cb = 0; cb < 4; cb++)
+			x[cb] = sa_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+		for (int s = 0; s < 16; s++)
+#pragma unroll
+			for (int cb = 0; cb < 4; cb++)
+				if (s < 4 * (cb + 1))
+					x[cb] = sa_mfma(Li[(16 * cb + r) + (4 * s + g) * LD], t[s], x[cb]);
+		__syncthreads();                 // L(j,j) has left S
+#pragma unroll
+		for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+			for (int q = 0; q < 4; q++) {
+				const int c = 16 * cb + 4 * q + g;
+				S[row + c * LD] = x[cb][q];
+				if (row < wn)
+					P[row + (long)c * p.lda] = x[cb][q];
+			}
+		__syncthreads();                 // S is whole
+		sa_d4 acc[3];
+#pragma unroll
+		for (int u = 0; u < 3; u++) {
+			const int b = 4 * u + wave, I = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, K = b - I * (I + 1) / 2;
+			acc[u] = sa_d4{0.0, 0.0, 0.0, 0.0};
+			if (b < 10)
+#pragma unroll
+				for (int s = 0; s < 16; s++)
+					acc[u] = sa_mfma(S[16 * K + r + (4 * s + g) * LD], S[16 * I + r + (4 * s + g) * LD], acc[u]);
+		}
+		publish(p.rowl(j + 1), (unsigned)j + 1);     // with a barrier: L(j+1,j) has left S
+#pragma unroll
+		for (int u = 0; u < 3; u++) {
+			const int b = 4 * u + wave, I = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, K = b - I * (I + 1) / 2;
+			if (b < 10)
+#pragma unroll
+				for (int q = 0; q < 4; q++) {
+					const int ic = 16 * I + r, jc = 16 * K + 4 * q + g;
+					S[ic + jc * LD] = (ic < wn && jc < wn) ? cv[u][q] - acc[u][q] : ic == jc ? 1.0 : 0.0;
+				}
+		}
+		__syncthreads();
+	}
 	if (threadIdx.x == 0)
-		*p.info = first_bad;
+		*p.info = flag_read(p.abortf()) ? -1 : first_bad;
 }
 
 // ---- the bulk order --------------------------------------------------------
-// Step s: P(a, s) for a = s+2..nb-1 and U(b, a, s) for a = s+1..nb-1,
-// b = a..nb-1 without the chain's (s+1, s+1) (factorisation, s < nb), then
-// for t = s - delay: WD(t), WX(j, t) for j < t (inverse).  Without the factorisation, step 0 starts with D(a), a < nb.
+// Step s: S(s) and G(s) (1 <= s < nb - 1), P(a, s) for a = s+2..nb-1
+// (factorisation, s < nb), then for t = s - delay: WD(t), WX(a, t) for a < t
+// (inverse).  Without the factorisation, step 0 starts with D(a), a < nb.
 // Host and device walk it with the same code (the host counts the items).
 
-enum { PH_D = 0, PH_P, PH_U, PH_WD, PH_WX, PH_END };
+enum { PH_D = 0, PH_S, PH_G, PH_P, PH_WD, PH_WX, PH_END };
 
 struct PfOrder {
 	int nb, factor, inv, delay;
 };
 
 struct Cursor {
-	int s, ph, a, b;
+	int s, ph, a;
 };
 
-__host__ __device__ inline bool phase_on(const PfOrder &o, int s, int ph)
+// First a of a phase of step s, and the one after its last (none if not above).
+__host__ __device__ inline int phase_first(const PfOrder &, int s, int ph) { return ph == PH_P ? s + 2 : 0; }
+
+__host__ __device__ inline int phase_last(const PfOrder &o, int s, int ph)
 {
 	const int t = s - o.delay;
 	switch (ph) {
 	case PH_D:
-		return !o.factor && s == 0;
+		return !o.factor && s == 0 ? o.nb : 0;
+	case PH_S:
+	case PH_G:
+		return o.factor && s >= 1 && s + 1 < o.nb ? 1 : 0;
 	case PH_P:
-	case PH_U:
-		return o.factor && s < o.nb;
+		return o.factor ? o.nb : 0;
+	case PH_WD:
+		return o.inv && t >= 0 && t < o.nb ? 1 : 0;
 	default:
-		return o.inv && t >= 0 && t < o.nb;
+		return o.inv && t < o.nb ? t : 0;
 	}
-}
-
-__host__ __device__ inline void phase_begin(Cursor &c, const PfOrder &o)
-{
-	(void)o;
-	c.a = c.b = 0;
-	if (c.ph == PH_P)
-		c.a = c.s + 2;
-	else if (c.ph == PH_U)
-		c.a = c.b = c.s + 1;
 }
 
 // Moves c to the first item at or after its position; false past the end.
 __host__ __device__ inline bool cursor_norm(Cursor &c, const PfOrder &o)
 {
 	const int last = o.nb - 1 + (o.factor && o.inv ? o.delay : 0);
-	for (;;) {
-		if (c.s > last)
-			return false;
-		if (c.ph >= PH_END) {
+	while (c.s <= last) {
+		if (c.a < phase_last(o, c.s, c.ph))
+			return true;
+		if (++c.ph >= PH_END) {
 			c.s++;
 			c.ph = 0;
-			phase_begin(c, o);
-			continue;
 		}
-		if (phase_on(o, c.s, c.ph)) {
-			const int s = c.s, t = s - o.delay;
-			switch (c.ph) {
-			case PH_D:
-			case PH_P:
-				if (c.a < o.nb)
-					return true;
-				break;
-			case PH_U:
-				if (c.a < o.nb) {
-					if (c.b >= o.nb) {
-						c.a++;
-						c.b = c.a;
-						continue;
-					}
-					if (c.a == s + 1 && c.b == s + 1) {
-						c.b++;
-						continue;
-					}
-					return true;
-				}
-				break;
-			case PH_WD:
-				if (c.a < 1)
-					return true;
-				break;
-			case PH_WX:
-				if (c.a < t)
-					return true;
-				break;
-			}
-		}
-		c.ph++;
-		phase_begin(c, o);
+		c.a = phase_first(o, c.s, c.ph);
 	}
-}
-
-__host__ __device__ inline void cursor_next(Cursor &c)
-{
-	if (c.ph == PH_U)
-		c.b++;
-	else
-		c.a++;
+	return false;
 }
 
 __host__ __device__ inline Cursor cursor_first(const PfOrder &o, bool *valid)
 {
-	Cursor c = {0, 0, 0, 0};
-	phase_begin(c, o);
+	Cursor c = {0, 0, 0};
 	*valid = cursor_norm(c, o);
 	return c;
 }
@@ -497,36 +630,38 @@ __device__ void run_bulk(const PfArgs &p, double *S, double *Li, int *s_ticket)
 	const PfOrder o = {p.nb, p.factor, p.inv, p.delay};
 	bool valid;
 	Cursor c = cursor_first(o, &valid);
-	int pos = 0, unused = 0;
+	int pos = 0;
 	for (;;) {
+		__syncthreads();                  // the last item's reads of LDS are done
 		if (threadIdx.x == 0)
-			*s_ticket = (int)atomicAdd(p.ticket, 1u);
+			*s_ticket = (int)atomicAdd(p.ticket(), 1u);
 		__syncthreads();
 		const int t = *s_ticket;
-		__syncthreads();
 		while (valid && pos < t) {
-			cursor_next(c);
+			c.a++;
 			valid = cursor_norm(c, o);
 			pos++;
 		}
-		if (!valid || aborted(p))
+		if (!valid)
 			break;                        // past the last item: this workgroup is done
-		const int s = c.s, ts = c.s - p.delay;
 		switch (c.ph) {
 		case PH_D:
-			item_D<false>(p, c.a, S, Li, unused);
+			item_D(p, c.a, S, Li);
+			break;
+		case PH_S:
+			item_prepare(p, c.s, c.s);
+			break;
+		case PH_G:
+			item_prepare(p, c.s, c.s + 1);
 			break;
 		case PH_P:
-			item_P(p, c.a, s);
-			break;
-		case PH_U:
-			item_U(p, c.b, c.a, s);
+			item_P(p, c.a, c.s, S);
 			break;
 		case PH_WD:
-			item_WD(p, ts);
+			item_WD(p, c.s - p.delay);
 			break;
 		default:
-			item_WX(p, c.a, ts);
+			item_WX(p, c.a, c.s - p.delay, S, Li);
 			break;
 		}
 	}
@@ -544,33 +679,31 @@ void k_potrf_tile(PfArgs p)
 		run_bulk(p, S, Li, &s_ticket);
 }
 
-// Counters of a launch: those of A's blocks zero when the tile is factored
-// here; when it is factored already, the off-diagonal blocks of L are final
-// (count l + 1) and the diagonal ones wait for their D item.  W's counters,
-// the ticket and the abort flag zero.  A kernel, not a memset, so that a
-// captured graph replays it correctly.
-__global__ void k_init_counters(unsigned *fa, unsigned *fw, int nb, int factor)
+// Counters of a launch.  When the tile is factored already, every row of L
+// is final.  Nothing has to be prepared for A(1,0) and A(1,1).  A kernel, not
+// a memset, so that a captured graph replays it correctly.
+__global__ void k_init_counters(unsigned *flags, int nb, int factor)
 {
-	for (int idx = threadIdx.x; idx < nb * nb; idx += blockDim.x) {
-		const int i = idx % nb, l = idx / nb;
-		fa[idx] = (!factor && i > l) ? (unsigned)l + 1 : 0u;
-		fw[idx] = 0u;
-	}
-	if (threadIdx.x == 0) {
-		fa[nb * nb] = 0u;       // ticket
-		fa[nb * nb + 1] = 0u;   // abort
+	for (int idx = threadIdx.x; idx < flag_words(nb); idx += blockDim.x) {
+		const int b = idx / FLAG_STRIDE;
+		unsigned v = 0u;
+		if (idx % FLAG_STRIDE == 0 && nb > 1) {     // one block: nothing waits
+			if (b < nb)
+				v = factor ? 0u : (unsigned)nb;     // rows of L
+			else if (b == nb + 1 || b == 2 * nb)
+				v = 1u;                             // diag(1), sub(0)
+		}
+		flags[idx] = v;
 	}
 }
 
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Workspace of a tile: the 64x64 block inverses, A's block counters with
-// the ticket and the abort flag, W's block counters.
+// Workspace of a tile: the 64x64 block inverses and the counters.
 constexpr size_t tile_bytes(int n)
 {
 	return align256((size_t)(n > 0 ? (n + 63) / 64 : 1) * 4096 * sizeof(double)) +
-	       align256(((size_t)(n > 0 ? (n + 63) / 64 : 1) * (n > 0 ? (n + 63) / 64 : 1) + 2) * sizeof(unsigned)) +
-	       align256((size_t)(n > 0 ? (n + 63) / 64 : 1) * (n > 0 ? (n + 63) / 64 : 1) * sizeof(unsigned));
+	       align256((size_t)flag_words(n > 0 ? (n + 63) / 64 : 1) * sizeof(unsigned));
 }
 
 long count_items(const PfOrder &o)
@@ -580,7 +713,7 @@ long count_items(const PfOrder &o)
 	long k = 0;
 	while (valid) {
 		k++;
-		cursor_next(c);
+		c.a++;
 		valid = cursor_norm(c, o);
 	}
 	return k;
@@ -606,20 +739,15 @@ int launch_tile(hipStream_t s, int n, double *A, int lda, int *dev_info, void *w
 	p.ldw = ldw;
 	p.Linv = Linv;
 	p.ldi = ldi;
-	const size_t dinv = align256((size_t)(nb ? nb : 1) * 4096 * sizeof(double));
-	const size_t cnt = align256(((size_t)(nb ? nb : 1) * (nb ? nb : 1) + 2) * sizeof(unsigned));
 	p.Dinv = (double *)ws;
-	p.fa = (unsigned *)(ws + dinv);
-	p.ticket = p.fa + (long)nb * nb;
-	p.abort = p.ticket + 1;
-	p.fw = (unsigned *)(ws + dinv + cnt);
+	p.flags = (unsigned *)(ws + align256((size_t)(nb ? nb : 1) * 4096 * sizeof(double)));
 	p.info = dev_info;
 	if (nb == 0) {
 		if (!factor)
 			return 0;
 		// n = 0: reports info = 0
 		p.nbulk = 0;
-		hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(64), 0, s, p.fa, p.fw, 1, 1);
+		hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(64), 0, s, p.flags, 1, 1);
 		int e = sa_launch_status();
 		if (e)
 			return e;
@@ -629,7 +757,7 @@ int launch_tile(hipStream_t s, int n, double *A, int lda, int *dev_info, void *w
 	const long items = count_items(PfOrder{nb, factor, p.inv, p.delay});
 	const int want = bulk > 0 ? (bulk < 255 ? bulk : 255) : max_bulk();
 	p.nbulk = (int)(items < want ? items : want);
-	hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(256), 0, s, p.fa, p.fw, nb, factor);
+	hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(256), 0, s, p.flags, nb, factor);
 	int e = sa_launch_status();
 	if (e)
 		return e;

@@ -309,6 +309,30 @@ def test_dpotrf_tile_factor_and_inverse_match_oracle(K, n):
     assert np.array_equal(dW3.download(), W) and np.array_equal(dA3.download(), got)
 
 
+@pytest.mark.parametrize("wg", [1, 255])
+@pytest.mark.parametrize("n", [63, 127, 128, 129, 190, 513])
+def test_dpotrf_tile_block_edges(K, n, wg):
+    # two, three and more block columns with full and ragged last blocks, odd
+    # leading dimensions, one bulk workgroup (every item in the fixed order)
+    # and more workgroups than items; factor alone and with the inverse give
+    # the same L.  Bars as the test above (n eps times a condition of ~5).
+    print(f"dpotrf_tile edges n={n} workgroups={wg}", flush=True)
+    rng = np.random.default_rng(7 * n + wg)
+    A = spd(rng, n)
+    ref = np.tril(oracle.dpotrf_l(A)[0])
+    dA, dA2 = K.DeviceArray.from_host(A, ld=n + 3), K.DeviceArray.from_host(A, ld=n + 3)
+    dX, dW = K.DeviceArray(n, n, ld=n + 1), K.DeviceArray(n, n, ld=n + 5)
+    info = K.DeviceInt(-7)
+    K.dpotrf_tile(n, dA.ptr, dA.ld, dX.ptr, dX.ld, dW.ptr, dW.ld, info.ptr, workgroups=wg)
+    assert info.get() == 0
+    got, X, W = dA.download(), dX.download(), dW.download()
+    iu = np.triu_indices(n, 1)
+    assert oracle.rel_diff_lower(np.tril(got), ref) < 1e-13 and np.array_equal(got[iu], A[iu])
+    assert rel(W, solve_triangular(ref, np.eye(n), lower=True).T) < 1e-13 and np.array_equal(X, W.T)
+    K.dpotrf_tile(n, dA2.ptr, dA2.ld, None, 0, None, 0, info.ptr, workgroups=wg)
+    assert info.get() == 0 and np.array_equal(dA2.download(), got)
+
+
 def test_tile_limit_and_large_tile_inverse(K):
     # tiles past the single-launch limit: sa_dpotrf_tile refuses them, and
     # sa_dtrtri_tile inverts them by substitution
