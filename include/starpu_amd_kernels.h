@@ -49,7 +49,9 @@ int sa_set_gemm_shape(int edge);
 
 /* Workgroup tile edge (64 or 128) that sa_dgemm_nt (lower = 0) or
  * sa_dsyrk_ln / the lower-triangle update (lower = 1, n ignored) would run
- * an m x n product with now; -EINVAL for an empty shape. */
+ * an m x n product with now; -EINVAL for an empty shape.  (64 stands for the
+ * kernel of single tile products, which takes 32x32 workgroups where 64x64
+ * ones would leave compute units idle.) */
 int sa_gemm_tile_shape(int lower, int m, int n);
 
 /* C(m x n) <- beta*C + alpha * A(m x k) * B(n x k)^T.

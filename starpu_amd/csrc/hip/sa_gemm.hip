@@ -1,19 +1,15 @@
 // FP64 GEMM NT and SYRK (lower) on the CDNA matrix cores (gfx950).
 //
 // C = beta*C + alpha*A*B^T with A (m x k), B (n x k), C (m x n), column-major.
-// Each wave owns a (16*WB) x (16*WB) block of C as WB x WB tiles of
-// v_mfma_f64_16x16x4f64; a workgroup has WVM x WVN waves.  Rows inside a
-// wave are interleaved (MFMA tile b, MFMA row r -> C row WB*r + b) so each
-// lane's A and B fragments for one k are WB contiguous doubles (16-byte
-// loads) and its C values come in WB-row runs.  Operands stream from L2
-// straight into registers through a two-stage register pipeline; stages
-// past k load clamped addresses and are zeroed with selects, so the loop
-// body has no branches and the accumulators stay in AGPRs.
+// Two kernels on v_mfma_f64_16x16x4f64:
 //
-// Two shapes are built: 64x64 waves in 128x128 workgroups (large problems,
-// two workgroups per compute unit) and 32x32 waves in 64x64 workgroups,
-// which gives a 1024x1024 tile 256 workgroups -- one per compute unit -- so
-// a single tile GEMM fills the GPU.
+// k_dgemm_lds  workgroup tiles of 64x64 or 32x32, operands staged in LDS: a
+//              single tile product (a tile task alone, or a few of them in
+//              flight), any size, alignment and leading dimension.
+// k_dgemm_nt   128x128 workgroup tiles (64x64 waves), operands from L2
+//              straight into registers: large products, and many tile
+//              products in flight, where two workgroups share a compute unit.
+
 #include <atomic>
 
 #include "sa_common.h"
@@ -21,6 +17,14 @@
 
 namespace {
 
+// k_dgemm_nt: each wave owns a (16*WB) x (16*WB) block of C as WB x WB MFMA
+// tiles; a workgroup has WVM x WVN waves.  Rows inside a wave are
+// interleaved (MFMA tile b, MFMA row r -> C row WB*r + b) so each lane's A
+// and B fragments for one k are WB contiguous doubles (16-byte loads) and
+// its C values come in WB-row runs.  Operands stream from L2 straight into
+// registers through a two-stage register pipeline; stages past k load
+// clamped addresses and are zeroed with selects, so the loop body has no
+// branches and the accumulators stay in AGPRs.
 template <bool EDGE, int WB>
 __device__ __forceinline__ void loadw(double (&v)[WB], const double *__restrict__ X, long ld,
                                       int row, int nrows, int k, int K)
@@ -175,6 +179,214 @@ void k_dgemm_nt(int M, int N, int K, double alpha, const double *__restrict__ A,
 	}
 }
 
+// The LDS-staged form: workgroup tiles of 32 WB x 32 WB (2 x 2 waves, each a
+// (16 WB) x (16 WB) block).  The operand panels go through registers into
+// LDS KC columns at a time: a thread loads single elements (64 or 32
+// consecutive rows per column, so a wave's load is whole lines whatever the
+// alignment), PF chunks ahead of their use, and each operand element is read
+// from the cache once per workgroup instead of once per wave.  Rows past the
+// matrix are read from its last row and not stored, columns k >= K are zero.
+// Two LDS buffers, one barrier a chunk.  C is loaded at the start, ahead of
+// everything that needs it.  The MFMA computes the transposed block, so that
+// a lane's values of C are in consecutive lanes' rows: acc[j][i][q] =
+// C(16 i + r, 16 j + 4q + g) of the wave's block.  The terms are added in the
+// order of k, as in k_dgemm_nt.
+//
+// Bound: the MFMAs, and before that a wave's in-order issue.  There is
+// mostly one wave per SIMD, whose LDS and memory instructions cost their
+// issue and wait unless MFMAs stand between them: with the same loads,
+// stores and MFMAs in three groups per chunk a 512^3 product took 31 us,
+// interleaved one by one 22 (64x64 tiles; 20 with the MFMAs alone).  Alone /
+// four in flight (us each): 256^3 6.1 / 4.5 with 32x32 tiles; 500^3 with
+// an odd leading dimension 9.8 / 7.4; 512^3 9.4 / 6.9; 960^3 39.9 / 33.8 and
+// 1024^3 42.7 / 36.8 with 64x64 tiles (58 TFLOP/s).  The same products took
+// 15.0 / 8.0, 40.0 / 24.6, 25.8 / 16.3, 48.9 / 40.5 and 50.7 / 42.7 with
+// 64x64 workgroups on k_dgemm_nt's register pipeline, where every wave loads
+// its own operands.
+template <int WB, int KC, int PF, bool LOWER, bool BETA0>
+__global__ __launch_bounds__(256)
+void k_dgemm_lds(int M, int N, int K, double alpha, const double *__restrict__ A, long lda,
+                 const double *__restrict__ B, long ldb, double beta, double *__restrict__ C, long ldc,
+                 int tiles_m, int ktri)
+{
+	constexpr int BT = 32 * WB, WT = 16 * WB;
+	constexpr int KSTEP = 256 / BT;           // columns one load of all threads covers
+	constexpr int NL = KC / KSTEP;            // loads per thread, operand and chunk
+	constexpr int LDT = BT + 16;              // LDS row: the four columns of an MFMA step in different banks
+	static_assert(PF % 2 == 0, "a chunk's LDS buffer follows from its register stage");
+	__shared__ double As[2][KC * LDT], Bs[2][KC * LDT];
+	int tm, tn;
+	if (LOWER) {
+		const int t = blockIdx.x;
+		int i = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+		while ((i + 1) * (i + 2) / 2 <= t) i++;
+		while (i * (i + 1) / 2 > t) i--;
+		tm = i;
+		tn = t - i * (i + 1) / 2;
+	} else {
+		// tile order as k_dgemm_nt: near-square groups per XCD
+		int t = blockIdx.x;
+		const int T = gridDim.x;
+		if ((T & 7) == 0)
+			t = (t & 7) * (T >> 3) + (t >> 3);
+		const int tiles_n = T / tiles_m;
+		int G = 1;
+		while (2 * G <= tiles_m && tiles_m % (2 * G) == 0 && 4 * G * G <= (T >> 3))
+			G *= 2;
+		tm = (t / (G * tiles_n)) * G + t % G;
+		tn = (t / G) % tiles_n;
+	}
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+	const int wr = (wave & 1) * WT, wc = (wave >> 1) * WT;
+	const int row0 = tm * BT + wr, col0 = tn * BT + wc;
+	// ktri: as k_dgemm_nt, here for the workgroup's columns together
+	if (ktri && tn * BT + BT < K)
+		K = tn * BT + BT;
+	const bool active = row0 < M && col0 < N && !(LOWER && row0 + WT <= col0);
+
+	double cv[WB][WB][4];
+	if (!BETA0 && active) {
+#pragma unroll
+		for (int j = 0; j < WB; j++)
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+#pragma unroll
+				for (int i = 0; i < WB; i++) {
+					const int row = row0 + 16 * i + r, col = col0 + 16 * j + 4 * q + g;
+						const int cc = col < N ? col : N - 1;
+					const int rc = row < M ? row : M - 1;
+					cv[j][i][q] = C[(LOWER && rc < cc ? cc : rc) + (long)cc * ldc];
+				}
+	}
+
+	// a thread's element of a chunk's load i: uniform base + its own offset
+	const int lr = tid % BT, lk = tid / BT;
+	const long oa = (tm * BT + lr < M ? lr : M - 1 - tm * BT) + lk * lda;
+	const long ob = (tn * BT + lr < N ? lr : N - 1 - tn * BT) + lk * ldb;
+	const double *A0 = A + tm * BT, *B0 = B + tn * BT;
+	const int nfull = K / KC, nch = (K + KC - 1) / KC;
+	double ra[PF][NL], rb[PF][NL];
+	// chunk c, or the last full one in place of those past it (never used)
+	auto load = [&](int c, double (&xa)[NL], double (&xb)[NL]) {
+		const long k = (long)(c < nfull ? c : nfull - 1) * KC;
+#pragma unroll
+		for (int i = 0; i < NL; i++) {
+			xa[i] = (A0 + (k + KSTEP * i) * lda)[oa];
+			xb[i] = (B0 + (k + KSTEP * i) * ldb)[ob];
+		}
+	};
+	auto store = [&](int buf, const double (&xa)[NL], const double (&xb)[NL]) {
+#pragma unroll
+		for (int i = 0; i < NL; i++) {
+			As[buf][(KSTEP * i + lk) * LDT + lr] = xa[i];
+			Bs[buf][(KSTEP * i + lk) * LDT + lr] = xb[i];
+		}
+	};
+	sa_d4 acc[WB][WB];
+#pragma unroll
+	for (int j = 0; j < WB; j++)
+#pragma unroll
+		for (int i = 0; i < WB; i++)
+			acc[j][i] = sa_d4{0.0, 0.0, 0.0, 0.0};
+	double fa[2][KC / 4][WB], fb[2][KC / 4][WB];
+	auto fetch = [&](int buf, double (&xa)[KC / 4][WB], double (&xb)[KC / 4][WB]) {
+#pragma unroll
+		for (int s = 0; s < KC / 4; s++)
+#pragma unroll
+			for (int i = 0; i < WB; i++) {
+				xa[s][i] = As[buf][(4 * s + g) * LDT + wr + 16 * i + r];
+				xb[s][i] = Bs[buf][(4 * s + g) * LDT + wc + 16 * i + r];
+			}
+	};
+	auto compute = [&](const double (&xa)[KC / 4][WB], const double (&xb)[KC / 4][WB]) {
+#pragma unroll
+		for (int s = 0; s < KC / 4; s++)
+#pragma unroll
+			for (int j = 0; j < WB; j++)
+#pragma unroll
+				for (int i = 0; i < WB; i++)
+					acc[j][i] = sa_mfma(xb[s][j], xa[s][i], acc[j][i]);
+	};
+	// One chunk: the MFMAs on its fragments, and between them, one by one,
+	// the LDS reads of the next chunk's, the LDS stores of the chunk after
+	// that and the loads of the chunk PF further on.  A wave issues in order
+	// and there is mostly one per SIMD, so memory instructions in a row
+	// would leave the matrix core idle.  No branch: what goes past the last
+	// full chunk repeats it and is not used.
+	auto step = [&](int c, int u) {
+		fetch((u + 1) & 1, fa[(u + 1) & 1], fb[(u + 1) & 1]);
+		store(u & 1, ra[(u + 2) % PF], rb[(u + 2) % PF]);
+		load(c + 2 + PF, ra[(u + 2) % PF], rb[(u + 2) % PF]);
+		compute(fa[u & 1], fb[u & 1]);
+		constexpr int NM = (KC / 4) * WB * WB;                     // MFMAs
+		constexpr int NR = (KC / 4) * WB, NS = 2 * NL;             // LDS reads (pairs), stores, loads
+#pragma unroll
+		for (int q = 0; q < NM; q++) {
+			__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+			// first half of the MFMAs: the reads; second half: stores, loads
+			const int h = NM / 2;
+			if (q < h) {
+				__builtin_amdgcn_sched_group_barrier(0x100, (NR + h - 1) / h, 0);
+			} else {
+				__builtin_amdgcn_sched_group_barrier(0x200, (NS + h - 1) / h, 0);
+				__builtin_amdgcn_sched_group_barrier(0x020, (NS + h - 1) / h, 0);
+			}
+		}
+		__builtin_amdgcn_sched_barrier(0);
+		__syncthreads();
+		__builtin_amdgcn_sched_barrier(0);
+	};
+	if (nfull > 0) {
+#pragma unroll
+		for (int u = 0; u < PF; u++)
+			load(u, ra[u], rb[u]);
+		store(0, ra[0], rb[0]);
+		load(PF, ra[0], rb[0]);
+		store(1, ra[1], rb[1]);
+		load(PF + 1, ra[1], rb[1]);
+		__syncthreads();
+		fetch(0, fa[0], fb[0]);
+		__syncthreads();
+		int c0 = 0;
+		for (; c0 + PF <= nfull; c0 += PF) {
+#pragma unroll
+			for (int u = 0; u < PF; u++)
+				step(c0 + u, u);
+		}
+#pragma unroll
+		for (int u = 0; u < PF - 1; u++)
+			if (c0 + u < nfull)
+				step(c0 + u, u);
+	}
+	if (nfull < nch) {
+		// the last K % KC columns, zero past K
+#pragma unroll
+		for (int i = 0; i < NL; i++) {
+			const int k = nfull * KC + KSTEP * i + lk;
+			const long back = k < K ? 0 : k - (K - 1);
+			const double xa = (A0 + (long)(nfull * KC + KSTEP * i) * lda)[oa - back * lda];
+			const double xb = (B0 + (long)(nfull * KC + KSTEP * i) * ldb)[ob - back * ldb];
+			As[0][(KSTEP * i + lk) * LDT + lr] = k < K ? xa : 0.0;
+			Bs[0][(KSTEP * i + lk) * LDT + lr] = k < K ? xb : 0.0;
+		}
+		__syncthreads();
+		fetch(0, fa[0], fb[0]);
+		compute(fa[0], fb[0]);
+	}
+	if (!active)
+		return;
+#pragma unroll
+	for (int j = 0; j < WB; j++)
+#pragma unroll
+		for (int q = 0; q < 4; q++)
+#pragma unroll
+			for (int i = 0; i < WB; i++) {
+				const int row = row0 + 16 * i + r, col = col0 + 16 * j + 4 * q + g;
+				if (row < M && col < N && (!LOWER || row >= col))
+					C[row + (long)col * ldc] = (BETA0 ? 0.0 : beta * cv[j][i][q]) + alpha * acc[j][i][q];
+			}
+}
+
 // X <- a*X over an m x n region (lower: only i >= j).
 __global__ void k_scale(int m, int n, double *X, long ld, double a, int lower)
 {
@@ -213,6 +425,22 @@ int gemm_shape(hipStream_t s, int m, int n, int k, double alpha, const double *A
 	return sa_launch_status();
 }
 
+template <int WB, int KC, int PF, bool LOWER>
+int gemm_lds(hipStream_t s, int m, int n, int k, double alpha, const double *A, int lda, const double *B, int ldb,
+             double beta, double *C, int ldc, int ktri)
+{
+	constexpr int BT = 32 * WB;
+	const int tiles_m = (m + BT - 1) / BT, tiles_n = (n + BT - 1) / BT;
+	const unsigned grid = LOWER ? (unsigned)(tiles_m * (tiles_m + 1) / 2) : (unsigned)(tiles_m * tiles_n);
+	if (beta == 0.0)
+		hipLaunchKernelGGL((k_dgemm_lds<WB, KC, PF, LOWER, true>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A,
+		                   (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
+	else
+		hipLaunchKernelGGL((k_dgemm_lds<WB, KC, PF, LOWER, false>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A,
+		                   (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
+	return sa_launch_status();
+}
+
 // Launches the caller keeps in flight on one device (sa_set_launch_concurrency).
 std::atomic<int> g_concurrency{1};
 
@@ -236,11 +464,11 @@ int tile_shape_override()
 // Workgroup tile edge (64 or 128) that a product of this shape runs with.
 // 128x128 workgroups (half the operand traffic per flop) while the
 // launches in flight together give every compute unit about 1.5 of them;
-// otherwise 64x64 workgroups (4x as many).  Alone, a 1024x1024 tile product
-// thus runs as 256 workgroups of 64x64 (40.6 TFLOP/s); with 12 streams of
-// such products in flight, 128x128 workgroups ran the N=32768 tile-1024
-// factorisation at 49.0 TFLOP/s against 44.9 with 64x64 (same machine, 16
-// hardware queues).
+// otherwise the LDS-staged kernel with smaller ones.  With 12 streams of
+// 1024^3 products in flight over 16 hardware queues, 128x128 workgroups run
+// the N=32768 tile-1024 factorisation at 57 TFLOP/s; with the four queues of
+// a default process, where a 128x128 launch is 64 workgroups, the 64x64
+// workgroups do better (36.8 us a product against 87).
 int pick_shape(bool lower, int m, int n)
 {
 	const int forced = tile_shape_override();
@@ -281,8 +509,17 @@ int gemm_launch(hipStream_t s, bool lower, int m, int n, int k, double alpha, co
 	if (shape == 128)
 		return lower ? gemm_shape<4, 2, 2, true, 2>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri)
 		             : gemm_shape<4, 2, 2, false, 2>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
-	return lower ? gemm_shape<2, 2, 8, true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri)
-	             : gemm_shape<2, 2, 8, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
+	// 32x32 workgroups where 64x64 ones would not reach most of the 256
+	// compute units: 4 times as many, a quarter of the MFMAs each.  Alone /
+	// four in flight (us), 32x32 against 64x64: 256^3 6.1 / 4.5 and 13.3 / 7.5;
+	// 512^3 (64 of the latter) 9.4 / 6.9 and 22.6 / 12.0; the lower 1024^3 (136)
+	// 33.8 / 26.1 and 41.2 / 28.1; 960^3 (225) 42.5 / 37.8 and 39.9 / 33.8.
+	const long t64m = (m + 63) / 64, t64n = (n + 63) / 64;
+	if ((lower ? t64m * (t64m + 1) / 2 : t64m * t64n) < 192)
+		return lower ? gemm_lds<1, 16, 4, true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri)
+		             : gemm_lds<1, 16, 4, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
+	return lower ? gemm_lds<2, 16, 2, true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri)
+	             : gemm_lds<2, 16, 2, false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
 }
 
 } // namespace

@@ -63,6 +63,34 @@ def test_dgemm_nt_matches_oracle(K, shape, m, n, k, alpha, beta):
     assert rel(got, exp) < 1e-13
 
 
+@pytest.mark.parametrize("m,n", [(31, 33), (65, 200), (897, 961), (1030, 1100)])
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 33, 47, 64, 129])
+def test_dgemm_nt_staged_chunk_edges(K, m, n, k):
+    # the LDS-staged kernel (both of its workgroup tiles) around its 16-column
+    # chunks and its pipeline depth, odd leading dimensions: integers, so that
+    # a repeated, skipped or misplaced column changes the exact result; the
+    # rows between m and ld stay as they are, and SYRK leaves the upper half
+    prev = K.set_gemm_shape(64)
+    try:
+        print(f"staged gemm m={m} n={n} k={k}", flush=True)
+        rng = np.random.default_rng(m + n + k)
+        A, B = rng.integers(-9, 10, (m, k)).astype(float), rng.integers(-9, 10, (n, k)).astype(float)
+        C0 = rng.integers(-64, 65, (m + 3, n)).astype(float)
+        dA, dB, dC = dev(K, A, m + 1), dev(K, B, n + 5), dev(K, C0)
+        K.dgemm_nt(m, n, k, -1.0, dA.ptr, dA.ld, dB.ptr, dB.ld, 2.0, dC.ptr, dC.ld)
+        got = dC.download()
+        assert np.array_equal(got[:m], 2.0 * C0[:m] - A @ B.T) and np.array_equal(got[m:], C0[m:])
+        q = 1300 if m > 1000 else m
+        A = rng.integers(-9, 10, (q, k)).astype(float)
+        S0 = rng.integers(-64, 65, (q, q)).astype(float)
+        dA, dS = dev(K, A, q + 1), dev(K, S0, q + 3)
+        K.dsyrk_ln(q, k, 1.0, dA.ptr, dA.ld, -1.0, dS.ptr, dS.ld)
+        got = dS.download()
+        assert np.array_equal(np.tril(got), np.tril(A @ A.T - S0)) and np.array_equal(np.triu(got, 1), np.triu(S0, 1))
+    finally:
+        K.set_gemm_shape(prev)
+
+
 def test_dgemm_nt_integer_inputs_bit_exact(K, shape):
     rng = np.random.default_rng(5)
     m, n, k = 256, 384, 512
