@@ -219,9 +219,9 @@ int sa_sgemm_tn(hipStream_t stream, int mode, int upper, int m, int n, int k,
 
 /* C(m x n) <- beta*C + alpha * U^T * B with U (m x m) upper triangular and
  * its strict lower part stored as zeros (the mixed TRSM's W_k = U_kk^-1):
- * sa_sgemm_tn with k = m, the k-range of each 128-row block of C stopped
- * at its last row where the staged kernels run (about half the products;
- * the terms left out are exact zeros). */
+ * sa_sgemm_tn with k = m, the k-range of each workgroup's rows of C stopped
+ * at their last one (about half the products; the terms left out are exact
+ * zeros). */
 int sa_sgemm_tn_utri(hipStream_t stream, int mode, int m, int n, float alpha, const float *U, int ldu,
                      const float *B, int ldb, float beta, float *C, int ldc);
 

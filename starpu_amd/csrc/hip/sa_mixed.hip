@@ -4,10 +4,9 @@
 // stored column-major.  Every trailing update then reads both operands
 // along k with unit stride -- U_km^T U_kn for C_mn -- which is the operand
 // layout the MFMA instructions want (8 consecutive k per lane for the BF16
-// 16x16x32 form), so operands stream from L2 straight into registers with
-// 16-byte loads and no LDS transpose.
+// 16x16x32 form): 16-byte loads, no LDS transpose.
 //
-// k_sgemm_tn<MODE>: C(m x n) = beta*C + alpha * A^T B, A (k x m) and
+// k_sgemm_lds<MODE>: C(m x n) = beta*C + alpha * A^T B, A (k x m) and
 //   B (k x n) FP32, FP32 accumulation:
 //   MODE_F32   v_mfma_f32_16x16x4_f32;
 //   MODE_BF16  v_mfma_f32_16x16x32_bf16 on bf16(A), bf16(B);
@@ -48,66 +47,45 @@ struct Frag<MODE_BF16X3> {
 	sa_bf8 h, l;
 };
 
-template <int MODE>
-__device__ __forceinline__ Frag<MODE> make_frag(const float (&x)[8])
-{
-	Frag<MODE> f;
-	if constexpr (MODE == MODE_F32) {
-#pragma unroll
-		for (int e = 0; e < 8; e++)
-			f.v[e] = x[e];
-	} else if constexpr (MODE == MODE_BF16) {
-#pragma unroll
-		for (int e = 0; e < 8; e++)
-			f.h[e] = (__bf16)x[e];
-	} else {
-#pragma unroll
-		for (int e = 0; e < 8; e++) {
-			const __bf16 h = (__bf16)x[e];
-			f.h[e] = h;
-			f.l[e] = (__bf16)(x[e] - (float)h);
-		}
-	}
-	return f;
-}
+// The LDS-staged product for any size, alignment and leading dimension:
+// workgroup tiles of 32 WB x 32 WB (2 x 2 waves, WB = 4: 64x64 per wave, WB =
+// 2: 32x32).  Per 32-wide k chunk a thread loads WB runs of 4 k per operand
+// (16-byte loads that need only the alignment of a float), converts them --
+// for the BF16 modes into bf16 planes, hi and for BF16x3 lo -- and stores
+// them column by column in LDS (80-byte column stride for bf16, 144 for
+// FP32: the 16-byte fragment reads of 8 consecutive columns take different
+// banks); the waves read their MFMA fragments from there, lane group g
+// holding k = 8g + e of the chunk.  Columns past the matrix are read from its
+// last column and not stored; the last K % 32 columns are zero-padded.
+// In BF16x3 the three terms go in the order lo hi, hi lo, hi hi per chunk.
+//
+// Chunk c's MFMAs run with the fragments already in registers, and between
+// them, in a fixed interleaving, go the LDS reads of chunk c + 1, the
+// conversion and LDS stores of chunk c + 2 and the loads of chunk c + 4: a
+// wave issues in order and there is one per SIMD, so what does not stand
+// between MFMAs stands beside them.  One barrier a chunk.  Products of 1024^3
+// alone (us): FP32 23.1, BF16x3 18.3, BF16 11.0; of 469^3: 13.1, 10.9, 7.8.
+// With loads, conversion and stores in groups around the MFMAs, 128x128
+// workgroups and a 16-byte alignment they took 76.4, 37.7 and 22.0; without
+// the alignment, operands straight from L2, 469^3 took 56.
+template <int MODE> struct StageT { typedef __bf16 type; static constexpr int planes = MODE == MODE_BF16X3 ? 2 : 1, col = 40; };
+template <> struct StageT<MODE_F32> { typedef float type; static constexpr int planes = 1, col = 36; };
 
-// Lane group g holds k = 8g + e of a 32-wide k chunk in element e of both
-// operand fragments; any fixed assignment of k to (g, e) gives the same
-// sum, as long as the two operands agree.
+typedef float sa_f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 sa_bf4 __attribute__((ext_vector_type(4)));
 
-// 8 consecutive k of column `col` starting at k0 + 8g; past K (or past the
-// last column) the values are zero.  The fast path is two 16-byte loads.
-template <bool EDGE>
-__device__ __forceinline__ void load8(float (&v)[8], const float *__restrict__ X, long ld, int col, int ncols,
-                                      int k, int K)
-{
-	if (!EDGE) {
-		const sa_f4 *p = reinterpret_cast<const sa_f4 *>(X + k + (long)col * ld);
-		const sa_f4 a = p[0], b = p[1];
-		v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-		v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-	} else {
-		const bool cin = col < ncols;
-		const long cc = (long)(cin ? col : ncols - 1) * ld;
-#pragma unroll
-		for (int e = 0; e < 8; e++) {
-			const bool in = cin && (k + e) < K;
-			const float t = X[(in ? k + e : 0) + cc];
-			v[e] = in ? t : 0.0f;
-		}
-	}
-}
-
-template <int MODE, int WB, bool UPPER, bool EDGE>
+template <int MODE, int WB, bool UPPER>
 __global__ __launch_bounds__(256)
-void k_sgemm_tn(int M, int N, int K, float alpha, const float *__restrict__ A, long lda,
-                const float *__restrict__ B, long ldb, float beta, float *__restrict__ C, long ldc, int tiles_m)
+void k_sgemm_lds(int M, int N, int K, float alpha, const float *__restrict__ A, long lda,
+                 const float *__restrict__ B, long ldb, float beta, float *__restrict__ C, long ldc, int tiles_m,
+                 int ktri)
 {
-	constexpr int WT = 16 * WB;      // wave tile
-	constexpr int BT = 2 * WT;       // workgroup tile: 2 x 2 waves
+	typedef typename StageT<MODE>::type T;
+	constexpr int NPL = StageT<MODE>::planes, COL = StageT<MODE>::col;
+	constexpr int BT = 32 * WB, WT = 16 * WB;
+	__shared__ __attribute__((aligned(16))) T Ls[2][2][NPL][BT * COL];
 	int tm, tn;
 	if (UPPER) {
-		// workgroup tiles on and above the diagonal, column by column
 		const int t = blockIdx.x;
 		int j = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
 		while ((j + 1) * (j + 2) / 2 <= t) j++;
@@ -115,109 +93,187 @@ void k_sgemm_tn(int M, int N, int K, float alpha, const float *__restrict__ A, l
 		tn = j;
 		tm = t - j * (j + 1) / 2;
 	} else {
-		// XCD-grouped tile order, as the FP64 tile GEMM
 		int t = blockIdx.x;
-		const int T = gridDim.x;
-		if ((T & 7) == 0)
-			t = (t & 7) * (T >> 3) + (t >> 3);
-		const int tiles_n = T / tiles_m;
+		const int G0 = gridDim.x;
+		if ((G0 & 7) == 0)
+			t = (t & 7) * (G0 >> 3) + (t >> 3);
+		const int tiles_n = G0 / tiles_m;
 		int G = 1;
-		while (2 * G <= tiles_m && tiles_m % (2 * G) == 0 && 4 * G * G <= (T >> 3))
+		while (2 * G <= tiles_m && tiles_m % (2 * G) == 0 && 4 * G * G <= (G0 >> 3))
 			G *= 2;
 		tm = (t / (G * tiles_n)) * G + t % G;
 		tn = (t / G) % tiles_n;
 	}
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	const int i0 = tm * BT + (wave & 1) * WT;    // rows of C = columns of A
-	const int j0 = tn * BT + (wave >> 1) * WT;   // columns of C = columns of B
-	if (UPPER && i0 >= j0 + WT)
-		return;                                   // wave tile strictly below the diagonal
-	if (EDGE && (i0 >= M || j0 >= N))
-		return;
-	const int r = lane & 15, g = lane >> 4;
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+	const int I0 = tm * BT, J0 = tn * BT;
+	const int iw = (wave & 1) * WT, jw = (wave >> 1) * WT;
+	// ktri: A (K x M) is upper triangular with zeros stored below its
+	// diagonal, so the tile's output rows take only k < I0 + BT (the terms
+	// left out are exact zeros)
+	if (ktri && I0 + BT < K)
+		K = I0 + BT;
+	const int nfull = K / 32;
 
-	sa_f4 acc[WB][WB];                           // acc[bj][bi]: block (C rows bi, C cols bj)
-	float xa[WB][8], xb[WB][8], na[WB][8], nb[WB][8];
-	auto load_chunk = [&](float (&fa)[WB][8], float (&fb)[WB][8], int k0) {
-		const int k = k0 + 8 * g;
-		const bool kin = k < K;
-		const int kc = kin ? k : 0;
+	// thread t loads columns (t >> 3) + 32 u, k offset 4 (t & 7), u < WB
+	const int lcol = tid >> 3, lk = (tid & 7) * 4;
+	const float *pa[WB], *pb[WB];
 #pragma unroll
-		for (int b = 0; b < WB; b++) {
-			load8<EDGE>(fa[b], A, lda, i0 + 16 * b + r, M, kc, EDGE ? (kin ? K : 0) : K);
-			load8<EDGE>(fb[b], B, ldb, j0 + 16 * b + r, N, kc, EDGE ? (kin ? K : 0) : K);
+	for (int u = 0; u < WB; u++) {
+		const int ca = I0 + lcol + 32 * u, cb = J0 + lcol + 32 * u;
+		pa[u] = A + (long)(ca < M ? ca : M - 1) * lda;
+		pb[u] = B + (long)(cb < N ? cb : N - 1) * ldb;
+	}
+	sa_f4 ra[2][WB], rb[2][WB];
+	// chunk c, or the last full one in place of those past it (never used)
+	auto load = [&](int c, sa_f4 (&xa)[WB], sa_f4 (&xb)[WB]) {
+		const int k = 32 * (c < nfull ? c : nfull - 1) + lk;
+#pragma unroll
+		for (int u = 0; u < WB; u++) {
+			xa[u] = *reinterpret_cast<const sa_f4u *>(pa[u] + k);
+			xb[u] = *reinterpret_cast<const sa_f4u *>(pb[u] + k);
 		}
 	};
-	auto compute_chunk = [&](const float (&fa)[WB][8], const float (&fb)[WB][8], bool first) {
-		Frag<MODE> ya[WB], yb[WB];
+	auto put = [&](int buf, int op, int u, sa_f4 x) {
+		T *p = &Ls[buf][op][0][(lcol + 32 * u) * COL + lk];
+		if constexpr (MODE == MODE_F32) {
+			*reinterpret_cast<sa_f4 *>(p) = x;
+		} else {
+			sa_bf4 h, l;
+#pragma unroll
+			for (int e = 0; e < 4; e++) {
+				h[e] = (__bf16)x[e];
+				if (NPL == 2)
+					l[e] = (__bf16)(x[e] - (float)h[e]);
+			}
+			*reinterpret_cast<sa_bf4 *>(p) = h;
+			if (NPL == 2)
+				*reinterpret_cast<sa_bf4 *>(p + (NPL - 1) * BT * COL) = l;
+		}
+	};
+	auto store = [&](int buf, const sa_f4 (&xa)[WB], const sa_f4 (&xb)[WB]) {
+#pragma unroll
+		for (int u = 0; u < WB; u++) {
+			put(buf, 0, u, xa[u]);
+			put(buf, 1, u, xb[u]);
+		}
+	};
+	Frag<MODE> fa[2][WB], fb[2][WB];
+	auto get = [&](int buf, int op, int col) {
+		Frag<MODE> f;
+		const T *p = &Ls[buf][op][0][col * COL + 8 * g];
+		if constexpr (MODE == MODE_F32) {
+			const sa_f4 x = *reinterpret_cast<const sa_f4 *>(p), y = *reinterpret_cast<const sa_f4 *>(p + 4);
+#pragma unroll
+			for (int e = 0; e < 4; e++) {
+				f.v[e] = x[e];
+				f.v[4 + e] = y[e];
+			}
+		} else {
+			f.h = *reinterpret_cast<const sa_bf8 *>(p);
+			if constexpr (MODE == MODE_BF16X3)
+				f.l = *reinterpret_cast<const sa_bf8 *>(p + BT * COL);
+		}
+		return f;
+	};
+	auto fetch = [&](int buf, Frag<MODE> (&xa)[WB], Frag<MODE> (&xb)[WB]) {
 #pragma unroll
 		for (int b = 0; b < WB; b++) {
-			ya[b] = make_frag<MODE>(fa[b]);
-			yb[b] = make_frag<MODE>(fb[b]);
+			xa[b] = get(buf, 0, iw + 16 * b + r);
+			xb[b] = get(buf, 1, jw + 16 * b + r);
 		}
-		// one term at a time across all WB x WB independent accumulators, so
-		// consecutive MFMAs never wait on each other's result
+	};
+	sa_f4 acc[WB][WB];
+#pragma unroll
+	for (int a = 0; a < WB; a++)
+#pragma unroll
+		for (int b = 0; b < WB; b++)
+			acc[a][b] = sa_f4{0.0f, 0.0f, 0.0f, 0.0f};
+	auto compute = [&](const Frag<MODE> (&xa)[WB], const Frag<MODE> (&xb)[WB]) {
+#define SA_TILES(D, L, R)                                                                          \
+	_Pragma("unroll") for (int bj = 0; bj < WB; bj++)                                              \
+	_Pragma("unroll") for (int bi = 0; bi < WB; bi++)                                              \
+		acc[bj][bi] = D(xb[bj].L, xa[bi].R, acc[bj][bi], 0, 0, 0)
 		if constexpr (MODE == MODE_F32) {
 #pragma unroll
 			for (int e = 0; e < 8; e++)
-#pragma unroll
-				for (int bj = 0; bj < WB; bj++)
-#pragma unroll
-					for (int bi = 0; bi < WB; bi++)
-						acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-						    yb[bj].v[e], ya[bi].v[e],
-						    (first && e == 0) ? sa_f4{0.0f, 0.0f, 0.0f, 0.0f} : acc[bj][bi], 0, 0, 0);
-		} else if constexpr (MODE == MODE_BF16) {
-#pragma unroll
-			for (int bj = 0; bj < WB; bj++)
-#pragma unroll
-				for (int bi = 0; bi < WB; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-					    yb[bj].h, ya[bi].h, first ? sa_f4{0.0f, 0.0f, 0.0f, 0.0f} : acc[bj][bi], 0, 0, 0);
+				SA_TILES(__builtin_amdgcn_mfma_f32_16x16x4f32, v[e], v[e]);
 		} else {
-#pragma unroll
-			for (int bj = 0; bj < WB; bj++)
-#pragma unroll
-				for (int bi = 0; bi < WB; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-					    yb[bj].l, ya[bi].h, first ? sa_f4{0.0f, 0.0f, 0.0f, 0.0f} : acc[bj][bi], 0, 0, 0);
-#pragma unroll
-			for (int bj = 0; bj < WB; bj++)
-#pragma unroll
-				for (int bi = 0; bi < WB; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(yb[bj].h, ya[bi].l, acc[bj][bi], 0, 0, 0);
-#pragma unroll
-			for (int bj = 0; bj < WB; bj++)
-#pragma unroll
-				for (int bi = 0; bi < WB; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(yb[bj].h, ya[bi].h, acc[bj][bi], 0, 0, 0);
+			if constexpr (MODE == MODE_BF16X3) {
+				SA_TILES(__builtin_amdgcn_mfma_f32_16x16x32_bf16, l, h);
+				SA_TILES(__builtin_amdgcn_mfma_f32_16x16x32_bf16, h, l);
+			}
+			SA_TILES(__builtin_amdgcn_mfma_f32_16x16x32_bf16, h, h);
 		}
+#undef SA_TILES
 	};
-
-	// two register stages: the next chunk loads while this one computes;
-	// the first chunk is peeled so the accumulators start from zero
-	load_chunk(xa, xb, 0);
-	if (32 < K)
-		load_chunk(na, nb, 32);
-	compute_chunk(xa, xb, true);
-	int k0 = 32;
-	while (k0 < K) {
-		if (k0 + 32 < K)
-			load_chunk(xa, xb, k0 + 32);
-		compute_chunk(na, nb, false);
-		k0 += 32;
-		if (k0 >= K)
-			break;
-		if (k0 + 32 < K)
-			load_chunk(na, nb, k0 + 32);
-		compute_chunk(xa, xb, false);
-		k0 += 32;
+	auto step = [&](int c, int u) {
+		fetch(u ^ 1, fa[u ^ 1], fb[u ^ 1]);
+		store(u, ra[u], rb[u]);
+		load(c + 4, ra[u], rb[u]);
+		compute(fa[u], fb[u]);
+		constexpr int NM = WB * WB * (MODE == MODE_F32 ? 8 : MODE == MODE_BF16X3 ? 3 : 1);   // MFMAs
+		constexpr int NR = 2 * WB * (MODE == MODE_BF16 ? 1 : 2);                             // LDS reads
+		constexpr int NS = 2 * WB * NPL, NG = 2 * WB;                                        // LDS stores, loads
+		constexpr int NV = MODE == MODE_F32 ? 0 : 2 * WB * (NPL == 2 ? 14 : 4);              // conversions, about
+		constexpr int H = NM / 3 > 0 ? NM / 3 : 1;
+#pragma unroll
+		for (int q = 0; q < NM; q++) {
+			__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+			if (NV)
+				__builtin_amdgcn_sched_group_barrier(0x002, (NV + NM - 1) / NM, 0);
+			if (q < H) {
+				__builtin_amdgcn_sched_group_barrier(0x100, (NR + H - 1) / H, 0);
+			} else if (q < 2 * H) {
+				__builtin_amdgcn_sched_group_barrier(0x200, (NS + H - 1) / H, 0);
+			} else if (q < 3 * H) {
+				__builtin_amdgcn_sched_group_barrier(0x200, (NS + H - 1) / H, 0);
+				__builtin_amdgcn_sched_group_barrier(0x020, (NG + H - 1) / H, 0);
+			}
+		}
+		__builtin_amdgcn_sched_barrier(0);
+		__syncthreads();
+		__builtin_amdgcn_sched_barrier(0);
+	};
+	if (nfull > 0) {
+		load(0, ra[0], rb[0]);
+		load(1, ra[1], rb[1]);
+		store(0, ra[0], rb[0]);
+		load(2, ra[0], rb[0]);
+		store(1, ra[1], rb[1]);
+		load(3, ra[1], rb[1]);
+		__syncthreads();
+		fetch(0, fa[0], fb[0]);
+		__syncthreads();
+		int c = 0;
+		for (; c + 2 <= nfull; c += 2) {
+			step(c, 0);
+			step(c + 1, 1);
+		}
+		if (c < nfull)
+			step(c, 0);
 	}
-
-	// lane holds C(i0 + 16 bi + r, j0 + 16 bj + 4g + q) in acc[bj][bi][q].
-	// All C values are loaded first (clamped addresses, no branches), so the
-	// loads are in flight together; beta == 0 selects zero without reading
-	// anything into the result.
+	if (32 * nfull < K) {
+		// the last K % 32 columns, zero past K
+#pragma unroll
+		for (int u = 0; u < WB; u++) {
+			sa_f4 xa, xb;
+#pragma unroll
+			for (int e = 0; e < 4; e++) {
+				const int k = 32 * nfull + lk + e, kc = k < K ? k : K - 1;
+				const float va = pa[u][kc], vb = pb[u][kc];
+				xa[e] = k < K ? va : 0.0f;
+				xb[e] = k < K ? vb : 0.0f;
+			}
+			put(0, 0, u, xa);
+			put(0, 1, u, xb);
+		}
+		__syncthreads();
+		fetch(0, fa[0], fb[0]);
+		compute(fa[0], fb[0]);
+	}
+	if (I0 + iw >= M || J0 + jw >= N || (UPPER && I0 + iw >= J0 + jw + WT))
+		return;
+	// lane holds C(I0 + iw + 16 bi + r, J0 + jw + 16 bj + 4g + q) in acc[bj][bi][q]
 	float cv[WB][4][WB];
 #pragma unroll
 	for (int bj = 0; bj < WB; bj++)
@@ -225,389 +281,42 @@ void k_sgemm_tn(int M, int N, int K, float alpha, const float *__restrict__ A, l
 		for (int q = 0; q < 4; q++)
 #pragma unroll
 			for (int bi = 0; bi < WB; bi++) {
-				int jc = j0 + 16 * bj + 4 * g + q, ic = i0 + 16 * bi + r;
-				if (EDGE) {
-					jc = jc < N ? jc : N - 1;
-					ic = ic < M ? ic : M - 1;
-				}
-				cv[bj][q][bi] = C[ic + (long)jc * ldc];
+				const int ic = I0 + iw + 16 * bi + r, jc = J0 + jw + 16 * bj + 4 * g + q;
+				cv[bj][q][bi] = C[(ic < M ? ic : M - 1) + (long)(jc < N ? jc : N - 1) * ldc];
 			}
 #pragma unroll
 	for (int bj = 0; bj < WB; bj++)
 #pragma unroll
-		for (int q = 0; q < 4; q++) {
-			const int jc = j0 + 16 * bj + 4 * g + q;
+		for (int q = 0; q < 4; q++)
 #pragma unroll
 			for (int bi = 0; bi < WB; bi++) {
-				const int ic = i0 + 16 * bi + r;
+				const int ic = I0 + iw + 16 * bi + r, jc = J0 + jw + 16 * bj + 4 * g + q;
 				const float c0 = beta == 0.0f ? 0.0f : beta * cv[bj][q][bi];
-				const bool keep = !(EDGE && (jc >= N || ic >= M)) && !(UPPER && ic > jc);
-				if (keep)
+				if (ic < M && jc < N && !(UPPER && ic > jc))
 					C[ic + (long)jc * ldc] = c0 + alpha * acc[bj][bi][q];
 			}
-		}
 }
 
-// LDS-staged form for the BF16 modes on full 128x128 workgroup tiles: per
-// 32-wide k chunk the workgroup loads its A and B panels (128 columns x 32
-// k each) once with 16-byte loads, splits them into bf16 planes (hi, and
-// lo for BF16x3) and stores them column by column in LDS (80-byte column
-// stride, so the 16-byte fragment reads of a 16-lane group hit distinct
-// banks); the four waves (2x2, 64x64 each) then read their MFMA fragments
-// from LDS.  Each operand is thus fetched from L2 and converted once per
-// workgroup instead of once per wave.  Two LDS buffers: the next chunk is
-// loaded into registers while the MFMAs run on the current one, and
-// stored into the other buffer; one barrier per chunk.
-constexpr int LBT = 128;    // workgroup tile
+template <int MODE, int WB, bool UPPER>
+int sgemm_lds(hipStream_t s, int m, int n, int k, float alpha, const float *A, int lda, const float *B, int ldb,
+              float beta, float *C, int ldc, int ktri)
+{
+	constexpr int BT = 32 * WB;
+	const int tiles_m = (m + BT - 1) / BT, tiles_n = (n + BT - 1) / BT;
+	const unsigned grid = UPPER ? (unsigned)(tiles_n * (tiles_n + 1) / 2) : (unsigned)(tiles_m * tiles_n);
+	hipLaunchKernelGGL((k_sgemm_lds<MODE, WB, UPPER>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A, (long)lda, B,
+	                   (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
+	return sa_launch_status();
+}
+
+constexpr int LBT = 128;    // workgroup tile of the split-plane kernels
 constexpr int LCOL = 40;    // bf16 per staged column: 32 k + 8 padding
-
-typedef __bf16 sa_bf4 __attribute__((ext_vector_type(4)));
-
-template <int MODE, bool UPPER, int NBUF, int PF = 1>
-__global__ __launch_bounds__(256)
-void k_sgemm_tn_lds(int M, int N, int K, float alpha, const float *__restrict__ A, long lda,
-                    const float *__restrict__ B, long ldb, float beta, float *__restrict__ C, long ldc, int tiles_m,
-                    int ktri)
-{
-	constexpr int NPL = (MODE == MODE_BF16X3) ? 2 : 1;
-	__shared__ __attribute__((aligned(16))) __bf16 Ls[NBUF][2][NPL][LBT * LCOL];
-	int tm, tn;
-	if (UPPER) {
-		const int t = blockIdx.x;
-		int j = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
-		while ((j + 1) * (j + 2) / 2 <= t) j++;
-		while (j * (j + 1) / 2 > t) j--;
-		tn = j;
-		tm = t - j * (j + 1) / 2;
-	} else {
-		int t = blockIdx.x;
-		const int T = gridDim.x;
-		if ((T & 7) == 0)
-			t = (t & 7) * (T >> 3) + (t >> 3);
-		const int tiles_n = T / tiles_m;
-		int G = 1;
-		while (2 * G <= tiles_m && tiles_m % (2 * G) == 0 && 4 * G * G <= (T >> 3))
-			G *= 2;
-		tm = (t / (G * tiles_n)) * G + t % G;
-		tn = (t / G) % tiles_n;
-	}
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int r = lane & 15, g = lane >> 4;
-	const int I0 = tm * LBT, J0 = tn * LBT;
-	const int i0w = (wave & 1) * 64, j0w = (wave >> 1) * 64;
-	// on a diagonal tile of the upper form, the wave block strictly below
-	// the diagonal takes part in loads and barriers but computes nothing.
-	// (A run-time value in both forms: with compute() unconditional the
-	// compiler interleaves it with the staging and runs out of registers.)
-	const bool active = !(UPPER && I0 + i0w >= J0 + j0w + 64) && M > 0;
-	// ktri: A (K x M) is upper triangular with zeros stored below its
-	// diagonal, so output rows I0 .. I0+127 take only k < I0 + 128 (the
-	// terms left out are exact zeros)
-	if (ktri && I0 + LBT < K)
-		K = I0 + LBT;
-
-	// thread t loads columns (t >> 3) + 32u, k offset 4 (t & 7), u = 0..3
-	const int lcol = tid >> 3, lk = (tid & 7) * 4;
-	sa_f4 ra[4], rb[4], ra2[4], rb2[4];
-	auto load_into = [&](int k0, sa_f4 (&xa)[4], sa_f4 (&xb)[4]) {
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			xa[u] = *reinterpret_cast<const sa_f4 *>(A + (k0 + lk) + (long)(I0 + lcol + 32 * u) * lda);
-			xb[u] = *reinterpret_cast<const sa_f4 *>(B + (k0 + lk) + (long)(J0 + lcol + 32 * u) * ldb);
-		}
-	};
-	auto load_stage = [&](int k0) { load_into(k0, ra, rb); };
-	auto store_from = [&](int buf, const sa_f4 (&ra)[4], const sa_f4 (&rb)[4]) {
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			const int off = (lcol + 32 * u) * LCOL + lk;
-			sa_bf4 ha, hb, la, lb;
-#pragma unroll
-			for (int e = 0; e < 4; e++) {
-				const __bf16 xa = (__bf16)ra[u][e], xb = (__bf16)rb[u][e];
-				ha[e] = xa;
-				hb[e] = xb;
-				if (NPL == 2) {
-					la[e] = (__bf16)(ra[u][e] - (float)xa);
-					lb[e] = (__bf16)(rb[u][e] - (float)xb);
-				}
-			}
-			*reinterpret_cast<sa_bf4 *>(&Ls[buf][0][0][off]) = ha;
-			*reinterpret_cast<sa_bf4 *>(&Ls[buf][1][0][off]) = hb;
-			if (NPL == 2) {
-				*reinterpret_cast<sa_bf4 *>(&Ls[buf][0][NPL - 1][off]) = la;
-				*reinterpret_cast<sa_bf4 *>(&Ls[buf][1][NPL - 1][off]) = lb;
-			}
-		}
-	};
-	auto store_stage = [&](int buf) { store_from(buf, ra, rb); };
-	sa_f4 acc[4][4];
-#pragma unroll
-	for (int a = 0; a < 4; a++)
-#pragma unroll
-		for (int b = 0; b < 4; b++)
-			acc[a][b] = sa_f4{0.0f, 0.0f, 0.0f, 0.0f};
-	auto compute = [&](int buf) {
-		// the wave issuing MFMAs goes first while the other waves of the CU
-		// convert and stage the next chunk (+4-8 % on 1024-wide products)
-		__builtin_amdgcn_s_setprio(1);
-		sa_bf8 ah[4], bh[4], al[4], bl[4];
-#pragma unroll
-		for (int b = 0; b < 4; b++) {
-			const int oa = (i0w + 16 * b + r) * LCOL + 8 * g, ob = (j0w + 16 * b + r) * LCOL + 8 * g;
-			ah[b] = *reinterpret_cast<const sa_bf8 *>(&Ls[buf][0][0][oa]);
-			bh[b] = *reinterpret_cast<const sa_bf8 *>(&Ls[buf][1][0][ob]);
-			if (NPL == 2) {
-				al[b] = *reinterpret_cast<const sa_bf8 *>(&Ls[buf][0][NPL - 1][oa]);
-				bl[b] = *reinterpret_cast<const sa_bf8 *>(&Ls[buf][1][NPL - 1][ob]);
-			}
-		}
-		if (NPL == 2) {
-#pragma unroll
-			for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-				for (int bi = 0; bi < 4; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[bj], ah[bi], acc[bj][bi], 0, 0, 0);
-#pragma unroll
-			for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-				for (int bi = 0; bi < 4; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[bj], al[bi], acc[bj][bi], 0, 0, 0);
-		}
-#pragma unroll
-		for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-			for (int bi = 0; bi < 4; bi++)
-				acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[bj], ah[bi], acc[bj][bi], 0, 0, 0);
-		__builtin_amdgcn_s_setprio(0);
-	};
-
-	if constexpr (NBUF == 2 && PF == 2) {
-		// global loads two chunks ahead: chunk c + 2 is loaded into one
-		// register stage while chunk c is computed and chunk c + 1 (loaded
-		// a chunk earlier) is converted into the other LDS buffer, so a
-		// round trip to L2 or HBM has two chunks' MFMAs to hide behind.
-		// Two chunks per trip name the register stages statically.
-		const int nch = K / 32;
-		load_into(0, ra, rb);
-		if (nch > 1)
-			load_into(32, ra2, rb2);
-		store_from(0, ra, rb);
-		__syncthreads();
-		for (int c = 0; c < nch; c += 2) {
-			if (c + 2 < nch)
-				load_into(32 * (c + 2), ra, rb);
-			if (active)
-				compute(0);
-			if (c + 1 < nch)
-				store_from(1, ra2, rb2);
-			__syncthreads();
-			if (c + 1 >= nch)
-				break;
-			if (c + 3 < nch)
-				load_into(32 * (c + 3), ra2, rb2);
-			if (active)
-				compute(1);
-			if (c + 2 < nch)
-				store_from(0, ra, rb);
-			__syncthreads();
-		}
-	} else if constexpr (NBUF == 2) {
-		load_stage(0);
-		store_stage(0);
-		__syncthreads();
-		for (int k0 = 0; k0 < K; k0 += 32) {
-			const int cur = (k0 >> 5) & 1;
-			const bool more = k0 + 32 < K;
-			if (more)
-				load_stage(k0 + 32);
-			if (active)
-				compute(cur);
-			if (more)
-				store_stage(cur ^ 1);
-			__syncthreads();
-		}
-	} else {
-		// one LDS buffer (half the LDS, twice the resident workgroups): the
-		// next chunk's loads are in flight during the MFMAs, two barriers
-		// per chunk
-		load_stage(0);
-		for (int k0 = 0; k0 < K; k0 += 32) {
-			store_stage(0);
-			__syncthreads();
-			if (k0 + 32 < K)
-				load_stage(k0 + 32);
-			if (active)
-				compute(0);
-			__syncthreads();
-		}
-	}
-	if (!active)
-		return;
-	// lane holds C(I0 + i0w + 16 bi + r, J0 + j0w + 16 bj + 4g + q) in acc[bj][bi][q]
-	float cv[4][4][4];
-#pragma unroll
-	for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-		for (int q = 0; q < 4; q++)
-#pragma unroll
-			for (int bi = 0; bi < 4; bi++)
-				cv[bj][q][bi] = C[(I0 + i0w + 16 * bi + r) + (long)(J0 + j0w + 16 * bj + 4 * g + q) * ldc];
-#pragma unroll
-	for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-		for (int q = 0; q < 4; q++) {
-			const int jc = J0 + j0w + 16 * bj + 4 * g + q;
-#pragma unroll
-			for (int bi = 0; bi < 4; bi++) {
-				const int ic = I0 + i0w + 16 * bi + r;
-				const float c0 = beta == 0.0f ? 0.0f : beta * cv[bj][q][bi];
-				if (!(UPPER && ic > jc))
-					C[ic + (long)jc * ldc] = c0 + alpha * acc[bj][bi][q];
-			}
-		}
-}
-
-// LDS-staged form for FP32 (v_mfma_f32_16x16x4f32) on full 128x128
-// workgroup tiles, the same scheme as the BF16 form: per 32-wide k chunk the
-// workgroup loads its A and B panels (128 columns x 32 k) once with 16-byte
-// loads and stores them column by column in LDS as FP32 (34-float column
-// stride: the 16 lanes of a group read 16 columns at the same k, two floats
-// apart in the banks); the four waves (2x2, 64x64 each) take their MFMA
-// fragments from LDS, 8 k-steps of 4 per chunk.  Two LDS buffers (68 KB):
-// the next chunk is loaded into registers while the MFMAs run on the current
-// one; one barrier per chunk.
-constexpr int LCOLF = 34;   // floats per staged column: 32 k + 2 padding
-
-template <bool UPPER>
-__global__ __launch_bounds__(256)
-void k_sgemm_tn_lds_f32(int M, int N, int K, float alpha, const float *__restrict__ A, long lda,
-                        const float *__restrict__ B, long ldb, float beta, float *__restrict__ C, long ldc,
-                        int tiles_m, int ktri)
-{
-	__shared__ __attribute__((aligned(16))) float Lf[2][2][LBT * LCOLF];
-	int tm, tn;
-	if (UPPER) {
-		const int t = blockIdx.x;
-		int j = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
-		while ((j + 1) * (j + 2) / 2 <= t) j++;
-		while (j * (j + 1) / 2 > t) j--;
-		tn = j;
-		tm = t - j * (j + 1) / 2;
-	} else {
-		int t = blockIdx.x;
-		const int T = gridDim.x;
-		if ((T & 7) == 0)
-			t = (t & 7) * (T >> 3) + (t >> 3);
-		const int tiles_n = T / tiles_m;
-		int G = 1;
-		while (2 * G <= tiles_m && tiles_m % (2 * G) == 0 && 4 * G * G <= (T >> 3))
-			G *= 2;
-		tm = (t / (G * tiles_n)) * G + t % G;
-		tn = (t / G) % tiles_n;
-	}
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int r = lane & 15, g = lane >> 4;
-	const int I0 = tm * LBT, J0 = tn * LBT;
-	const int i0w = (wave & 1) * 64, j0w = (wave >> 1) * 64;
-	const bool active = !(UPPER && I0 + i0w >= J0 + j0w + 64);
-	// ktri: A (K x M) is upper triangular with zeros stored below its
-	// diagonal, so output rows I0 .. I0+127 take only k < I0 + 128 (the
-	// terms left out are exact zeros)
-	if (ktri && I0 + LBT < K)
-		K = I0 + LBT;
-
-	// thread t loads columns (t >> 3) + 32u, k offset 4 (t & 7), u = 0..3
-	const int lcol = tid >> 3, lk = (tid & 7) * 4;
-	sa_f4 ra[4], rb[4];
-	auto load_stage = [&](int k0) {
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			ra[u] = *reinterpret_cast<const sa_f4 *>(A + (k0 + lk) + (long)(I0 + lcol + 32 * u) * lda);
-			rb[u] = *reinterpret_cast<const sa_f4 *>(B + (k0 + lk) + (long)(J0 + lcol + 32 * u) * ldb);
-		}
-	};
-	auto store_stage = [&](int buf) {
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			const int off = (lcol + 32 * u) * LCOLF + lk;     // 8-byte aligned: two float2 stores
-			float *pa = &Lf[buf][0][off], *pb = &Lf[buf][1][off];
-			*reinterpret_cast<float2 *>(pa) = make_float2(ra[u][0], ra[u][1]);
-			*reinterpret_cast<float2 *>(pa + 2) = make_float2(ra[u][2], ra[u][3]);
-			*reinterpret_cast<float2 *>(pb) = make_float2(rb[u][0], rb[u][1]);
-			*reinterpret_cast<float2 *>(pb + 2) = make_float2(rb[u][2], rb[u][3]);
-		}
-	};
-	sa_f4 acc[4][4];
-#pragma unroll
-	for (int a = 0; a < 4; a++)
-#pragma unroll
-		for (int b = 0; b < 4; b++)
-			acc[a][b] = sa_f4{0.0f, 0.0f, 0.0f, 0.0f};
-	auto compute = [&](int buf) {
-		__builtin_amdgcn_s_setprio(1);
-#pragma unroll
-		for (int s = 0; s < 8; s++) {
-			float af[4], bf[4];
-#pragma unroll
-			for (int b = 0; b < 4; b++) {
-				af[b] = Lf[buf][0][(i0w + 16 * b + r) * LCOLF + 4 * s + g];
-				bf[b] = Lf[buf][1][(j0w + 16 * b + r) * LCOLF + 4 * s + g];
-			}
-#pragma unroll
-			for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-				for (int bi = 0; bi < 4; bi++)
-					acc[bj][bi] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[bj], af[bi], acc[bj][bi], 0, 0, 0);
-		}
-		__builtin_amdgcn_s_setprio(0);
-	};
-
-	load_stage(0);
-	store_stage(0);
-	__syncthreads();
-	for (int k0 = 0; k0 < K; k0 += 32) {
-		const int cur = (k0 >> 5) & 1;
-		const bool more = k0 + 32 < K;
-		if (more)
-			load_stage(k0 + 32);
-		if (active)
-			compute(cur);
-		if (more)
-			store_stage(cur ^ 1);
-		__syncthreads();
-	}
-	if (!active)
-		return;
-	// lane holds C(I0 + i0w + 16 bi + r, J0 + j0w + 16 bj + 4g + q) in acc[bj][bi][q]
-	float cv[4][4][4];
-#pragma unroll
-	for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-		for (int q = 0; q < 4; q++)
-#pragma unroll
-			for (int bi = 0; bi < 4; bi++)
-				cv[bj][q][bi] = C[(I0 + i0w + 16 * bi + r) + (long)(J0 + j0w + 16 * bj + 4 * g + q) * ldc];
-#pragma unroll
-	for (int bj = 0; bj < 4; bj++)
-#pragma unroll
-		for (int q = 0; q < 4; q++) {
-			const int jc = J0 + j0w + 16 * bj + 4 * g + q;
-#pragma unroll
-			for (int bi = 0; bi < 4; bi++) {
-				const int ic = I0 + i0w + 16 * bi + r;
-				const float c0 = beta == 0.0f ? 0.0f : beta * cv[bj][q][bi];
-				if (!(UPPER && ic > jc))
-					C[ic + (long)jc * ldc] = c0 + alpha * acc[bj][bi][q];
-			}
-		}
-}
 
 // BF16x3 form on operands split ahead of time: A and B arrive as bf16
 // planes hi = bf16(x), lo = bf16(x - hi), each laid out like the FP32
 // matrix (k-contiguous columns, same leading dimension), as k_split_bf16x2
-// writes them once per factor panel.  Same tiles, LDS layout, MFMA order and
-// epilogue as k_sgemm_tn_lds<MODE_BF16X3>, so the result is bit-identical;
+// writes them once per factor panel.  Same order of the products and the
+// same epilogue as k_sgemm_lds<MODE_BF16X3>, so the result is bit-identical;
 // the workgroup copies 16-byte runs of 8 k per plane into LDS instead of
 // loading FP32 and splitting it, which removes the conversion from every
 // product that reads the panel.
@@ -920,81 +629,19 @@ void k_split_bf16x2(int m, int n, const float *__restrict__ A, long lda, __bf16 
 	L[i + (long)j * ldh] = (__bf16)(x - (float)h);
 }
 
-template <int MODE, int WB, bool UPPER>
-int sgemm_launch(hipStream_t s, int m, int n, int k, float alpha, const float *A, int lda, const float *B,
-                 int ldb, float beta, float *C, int ldc)
-{
-	constexpr int BT = 32 * WB;
-	const int tiles_m = (m + BT - 1) / BT, tiles_n = (n + BT - 1) / BT;
-	const unsigned grid = UPPER ? (unsigned)(tiles_n * (tiles_n + 1) / 2) : (unsigned)(tiles_m * tiles_n);
-	const bool vec = sa_aligned16(A) && sa_aligned16(B) && (lda % 4 == 0) && (ldb % 4 == 0) && (k % 32 == 0);
-	if (vec && m % BT == 0 && n % BT == 0)
-		hipLaunchKernelGGL((k_sgemm_tn<MODE, WB, UPPER, false>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A,
-		                   (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m);
-	else
-		hipLaunchKernelGGL((k_sgemm_tn<MODE, WB, UPPER, true>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A,
-		                   (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m);
-	return sa_launch_status();
-}
-
-// LDS buffers of the staged kernel: 2 (default: the next chunk is stored
-// while this one computes, one barrier per chunk) or 1 (half the LDS, two
-// barriers per chunk; measured slower on 1024-wide tiles, 96 against 109
-// TFLOP/s); SA_SGEMM_LDS_BUFFERS=1 selects it, for tuning.
-int lds_buffers()
-{
-	static int v = 0;
-	if (v == 0) {
-		const char *e = getenv("SA_SGEMM_LDS_BUFFERS");
-		v = (e && atoi(e) == 1) ? 1 : 2;
-	}
-	return v;
-}
-
-// Chunks of k between a global load of the staged kernel and its use: 2
-// (default) or 1 (SA_SGEMM_PREFETCH=1, for tuning).  Both give the same bits.
-// (Three chunks, with a third register stage, measured the same speed.)
-int prefetch_distance()
-{
-	static int v = 0;
-	if (v == 0) {
-		const char *e = getenv("SA_SGEMM_PREFETCH");
-		v = (e && atoi(e) == 1) ? 1 : 2;
-	}
-	return v;
-}
-
+// 64x64 workgroup tiles up to products that give 192 workgroups of 128x128:
+// four times the workgroups, three on a compute unit (against one of
+// 128x128), which alone and with four launches in flight is the faster:
+// 1024^3 FP32 23.1 / 20.8 us against 67.9 / 35.0, BF16x3 18.3 / 13.9 against
+// 31.7 / 17.5.
 template <int MODE, bool UPPER>
 int sgemm_shape(hipStream_t s, int m, int n, int k, float alpha, const float *A, int lda, const float *B,
                 int ldb, float beta, float *C, int ldc, int ktri = 0)
 {
-	if (m % LBT == 0 && n % LBT == 0 && k % 32 == 0 && sa_aligned16(A) && sa_aligned16(B) && lda % 4 == 0 &&
-	    ldb % 4 == 0) {
-		const int tiles_m = m / LBT, tiles_n = n / LBT;
-		const unsigned grid = UPPER ? (unsigned)(tiles_n * (tiles_n + 1) / 2) : (unsigned)(tiles_m * tiles_n);
-		if constexpr (MODE == MODE_F32) {
-			hipLaunchKernelGGL((k_sgemm_tn_lds_f32<UPPER>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A, (long)lda,
-			                   B, (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
-			return sa_launch_status();
-		} else {
-			if (lds_buffers() == 1)
-				hipLaunchKernelGGL((k_sgemm_tn_lds<MODE, UPPER, 1>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A,
-				                   (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
-			else if (prefetch_distance() == 2)
-				hipLaunchKernelGGL((k_sgemm_tn_lds<MODE, UPPER, 2, 2>), dim3(grid), dim3(256), 0, s, m, n, k, alpha,
-				                   A, (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
-			else
-				hipLaunchKernelGGL((k_sgemm_tn_lds<MODE, UPPER, 2>), dim3(grid), dim3(256), 0, s, m, n, k, alpha, A,
-				                   (long)lda, B, (long)ldb, beta, C, (long)ldc, tiles_m, ktri);
-			return sa_launch_status();
-		}
-	}
-	// 128x128 workgroups (64x64 per wave) once they give every CU a
-	// workgroup, 64x64 below that
-	const long big = (long)((m + 127) / 128) * ((n + 127) / 128);
-	if (big >= 64)
-		return sgemm_launch<MODE, 4, UPPER>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-	return sgemm_launch<MODE, 2, UPPER>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+	const long tm = (m + 127) / 128, tn = (n + 127) / 128;
+	if ((UPPER ? tn * (tn + 1) / 2 : tm * tn) >= 192)
+		return sgemm_lds<MODE, 4, UPPER>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
+	return sgemm_lds<MODE, 2, UPPER>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
 }
 
 // Block (r, c), r >= c, that is the t-th of the lower triangle of a grid of

@@ -66,6 +66,31 @@ def test_sgemm_tn_integer_exact_and_upper_mask(K, mode):
     assert np.array_equal(got[il], C0[il])                    # strict lower part untouched
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("m,n", [(33, 31), (130, 257), (1793, 1793)])
+@pytest.mark.parametrize("k", [1, 31, 32, 33, 64, 95, 128, 161])
+def test_sgemm_tn_staged_chunk_edges(K, mode, m, n, k):
+    # both workgroup tiles around the 32-wide chunks and the pipeline depth,
+    # with leading dimensions that leave the columns aligned to a float only:
+    # integers exact in bf16, so a repeated, skipped or misplaced k changes
+    # the exact result; rows past m and, for upper, the lower half untouched
+    print(f"staged sgemm mode={mode} m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(m + n + 7 * k + mode)
+    A = rng.integers(-9, 10, (k, m)).astype(np.float32)
+    B = rng.integers(-9, 10, (k, n)).astype(np.float32)
+    C0 = rng.integers(-64, 65, (m + 3, n)).astype(np.float32)
+    dA, dB = K.DeviceArray.from_host(A, ld=k + 1), K.DeviceArray.from_host(B, ld=k + 3)
+    dC = K.DeviceArray.from_host(C0)
+    K.sgemm_tn(mode, 0, m, n, k, -1.0, dA.ptr, dA.ld, dB.ptr, dB.ld, 2.0, dC.ptr, dC.ld)
+    got = dC.download()
+    assert np.array_equal(got[:m], 2.0 * C0[:m] - A.T @ B) and np.array_equal(got[m:], C0[m:])
+    S0 = rng.integers(-64, 65, (m, m)).astype(np.float32)
+    dS = K.DeviceArray.from_host(S0, ld=m + 1)
+    K.sgemm_tn(mode, 1, m, m, k, 1.0, dA.ptr, dA.ld, dA.ptr, dA.ld, -1.0, dS.ptr, dS.ld)
+    got = dS.download()
+    assert np.array_equal(np.triu(got), np.triu(A.T @ A - S0)) and np.array_equal(np.tril(got, -1), np.tril(S0, -1))
+
+
 @pytest.mark.parametrize("upper,m,n,k", [(0, 1024, 1024, 1024), (1, 1024, 1024, 1024), (0, 512, 384, 96),
                                          (1, 256, 256, 64)])
 def test_bf16x3_split_planes_match_fp32_operands(K, upper, m, n, k):
