@@ -36,23 +36,26 @@ using namespace sa64;
 // of one system (n x n, ld n), by one 256-thread workgroup:
 //   A(j0:n, j0:j0+w) -= L(j0:n, 0:j0) L(j0:j0+w, 0:j0)^T
 // (lower part of the diagonal block only).  Rows in groups of 64 RB, wave
-// v taking the 16 RB rows from 16 RB v (RB = 2 or 4 for FP64, chosen by the
-// autotuner; 2 for FP32: with 4 the FP32 version spills within the 256
-// VGPRs of two workgroups per CU and runs 1.6x slower); K = j0 in chunks of
-// 64, the chunk of the panel's own rows L(j0:j0+w, kc:kc+64) staged in LDS
-// (Bs, 64 x LD) and shared by the four waves, the wave's rows streamed from
-// memory once per panel.  Each wave keeps a (16 RB)x64 block of MFMA
-// accumulators and computes the transposed block, so a lane's results are
-// consecutive rows.  The next chunk's staging loads and row operands are in
-// flight during the current chunk's MFMAs.
+// v taking the 16 RB rows from 16 RB v (RB = 2 or 4, for FP64 chosen by the
+// autotuner; 2 for FP32); K = j0 in chunks of 64, the chunk of the panel's
+// own rows L(j0:j0+w, kc:kc+64) staged in LDS (Bs, 64 x LD) and shared by the
+// four waves, the wave's rows streamed from memory once per panel.  Each wave
+// keeps a (16 RB)x64 block of MFMA accumulators and computes the transposed
+// block, so a lane's results are consecutive rows.  Rows past the matrix are
+// read from its last row and columns past the panel from its first; what they
+// give is not stored, so the loop has no branch.  A step's LDS fragments are
+// read during the step before it, the next chunk's row operands are loaded
+// into the registers the step frees, and the next chunk's panel rows at its
+// start.
 template <typename T, int RB>
-__device__ void wg_panel_update(int n, int j0, int w, T *__restrict__ A, T *__restrict__ Bs)
+__device__ __forceinline__ void wg_panel_update(int n, int j0, int w, T *__restrict__ A, T *__restrict__ Bs)
 {
 	typedef typename V4<T>::type V;
+	typedef __attribute__((address_space(1))) T G;
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+	const int pc = lane < w ? lane : 0;              // this lane's row of the panel's chunk
 	for (int rg = j0; rg < n; rg += 64 * RB) {
 		const int row0 = rg + 16 * RB * wave;
-		const bool active = row0 < n;
 		V acc[RB][4];
 #pragma unroll
 		for (int a = 0; a < RB; a++)
@@ -60,71 +63,76 @@ __device__ void wg_panel_update(int n, int j0, int w, T *__restrict__ A, T *__re
 			for (int b = 0; b < 4; b++)
 				acc[a][b] = zero4<T>();
 		// operands of the wave's rows for one chunk: bo[s][a] = L(row, kc + 4s + g)
-		int rc[RB];
+		const G *pr[RB];
 #pragma unroll
 		for (int a = 0; a < RB; a++)
-			rc[a] = (row0 + 16 * a + r) < n ? row0 + 16 * a + r : n - 1;
+			pr[a] = (const G *)A + ((row0 + 16 * a + r) < n ? row0 + 16 * a + r : n - 1) + (long)g * n;
+		const G *pp = (const G *)A + (j0 + pc) + (long)wave * n;
 		T nxt[16], bo[16][RB];
 #pragma unroll
-		for (int q = 0; q < 16; q++) {
-			const int c = (tid + 256 * q) & 63, k = (tid + 256 * q) >> 6;
-			nxt[q] = c < w ? A[(j0 + c) + (long)k * n] : T(0);
-		}
-		if (active)
+		for (int q = 0; q < 16; q++)
+			nxt[q] = pp[(long)(4 * q) * n];
 #pragma unroll
-			for (int s = 0; s < 16; s++)
+		for (int s = 0; s < 16; s++)
 #pragma unroll
-				for (int a = 0; a < RB; a++)
-					bo[s][a] = A[rc[a] + (long)(4 * s + g) * n];
+			for (int a = 0; a < RB; a++)
+				bo[s][a] = pr[a][(long)(4 * s) * n];
 		for (int kc = 0; kc < j0; kc += 64) {
 			__syncthreads();                 // the previous chunk's readers are done
 #pragma unroll
-			for (int q = 0; q < 16; q++) {
-				const int c = (tid + 256 * q) & 63, k = (tid + 256 * q) >> 6;
-				Bs[c + k * LD] = nxt[q];
-			}
+			for (int q = 0; q < 16; q++)
+				Bs[lane + (wave + 4 * q) * LD] = nxt[q];
 			__syncthreads();
-			const bool more = kc + 64 < j0;
-			if (more)
+			// the chunk after this one, or this one again after the last
+			const long ahead = (long)(kc + 64 < j0 ? 64 : 0) * n;
+			pp += ahead;
 #pragma unroll
-				for (int q = 0; q < 16; q++) {
-					const int c = (tid + 256 * q) & 63, k = (tid + 256 * q) >> 6;
-					nxt[q] = c < w ? A[(j0 + c) + (long)(kc + 64 + k) * n] : T(0);
-				}
-			if (active) {
-				// the next chunk's row operands load into the registers each
-				// k-step frees, while this chunk's MFMAs run
+			for (int a = 0; a < RB; a++)
+				pr[a] += ahead;
 #pragma unroll
-				for (int s = 0; s < 16; s++) {
-					const int k = 4 * s + g;
-					T ao[4];
+			for (int q = 0; q < 16; q++)
+				nxt[q] = pp[(long)(4 * q) * n];
+			T ao[2][4];
+#pragma unroll
+			for (int b = 0; b < 4; b++)
+				ao[0][b] = Bs[(16 * b + r) + g * LD];
+#pragma unroll
+			for (int s = 0; s < 16; s++) {
+				if (s < 15)
 #pragma unroll
 					for (int b = 0; b < 4; b++)
-						ao[b] = Bs[(16 * b + r) + k * LD];
+						ao[(s + 1) & 1][b] = Bs[(16 * b + r) + (4 * s + 4 + g) * LD];
 #pragma unroll
-					for (int a = 0; a < RB; a++)
+				for (int a = 0; a < RB; a++)
 #pragma unroll
-						for (int b = 0; b < 4; b++)
-							acc[a][b] = sa_mfma(ao[b], bo[s][a], acc[a][b]);
-					if (more)
+					for (int b = 0; b < 4; b++)
+						acc[a][b] = sa_mfma(ao[s & 1][b], bo[s][a], acc[a][b]);
 #pragma unroll
-						for (int a = 0; a < RB; a++)
-							bo[s][a] = A[rc[a] + (long)(kc + 64 + k) * n];
-				}
+				for (int a = 0; a < RB; a++)
+					bo[s][a] = pr[a][(long)(4 * s) * n];
 			}
 		}
 		// acc[a][b][q] = (L L^T)(row0 + 16a + r, j0 + 16b + drow(q, g))
-		if (active)
 #pragma unroll
-			for (int a = 0; a < RB; a++)
+		for (int a = 0; a < RB; a++) {
+			const int row = row0 + 16 * a + r;
+			T cv[4][4];
 #pragma unroll
-				for (int b = 0; b < 4; b++)
+			for (int b = 0; b < 4; b++)
 #pragma unroll
-					for (int q = 0; q < 4; q++) {
-						const int row = row0 + 16 * a + r, c = 16 * b + drow<T>(q, g);
-						if (row < n && c < w && row - j0 >= c)
-							A[row + (long)(j0 + c) * n] -= acc[a][b][q];
-					}
+				for (int q = 0; q < 4; q++) {
+					const int c = 16 * b + drow<T>(q, g);
+					cv[b][q] = A[(row < n ? row : n - 1) + (long)(j0 + (c < w ? c : 0)) * n];
+				}
+#pragma unroll
+			for (int b = 0; b < 4; b++)
+#pragma unroll
+				for (int q = 0; q < 4; q++) {
+					const int c = 16 * b + drow<T>(q, g);
+					if (row < n && c < w && row - j0 >= c)
+						A[row + (long)(j0 + c) * n] = cv[b][q] - acc[a][b][q];
+				}
+		}
 	}
 }
 
@@ -277,7 +285,7 @@ __device__ __forceinline__ void solve_core(int n, const T *__restrict__ L, long 
 // solve_core with x held in LDS for n <= 1024 (one copy in, one copy out),
 // in global memory beyond.
 template <typename T>
-__device__ __noinline__ void wg_solve1(int n, const T *__restrict__ L, long ldl, const T *__restrict__ Dinv,
+__device__ __forceinline__ void wg_solve1(int n, const T *__restrict__ L, long ldl, const T *__restrict__ Dinv,
                                        T *__restrict__ x, T *__restrict__ Tl)
 {
 	__shared__ T xs[1024];
@@ -294,28 +302,30 @@ __device__ __noinline__ void wg_solve1(int n, const T *__restrict__ L, long ldl,
 	}
 }
 
-// Out-of-line steps of the factorisation: each gets its own register
-// allocation, which keeps the FP32 refinement kernel within the 256 VGPRs
-// of two resident workgroups per CU and the FP64 panel update free of
-// spills.  (The FP64 kernel inlines the block factor and the panel apply:
-// the block factor alone needs ~360 VGPRs.)
-template <typename T>
-__device__ __noinline__ int nb_block_potrf(int w, T *D, long ldd, T *Dinv, T *S, T *Li)
+// Out-of-line steps of the FP32 kernel: each gets its own register
+// allocation, which keeps it within the 256 VGPRs of two resident workgroups
+// per CU.  Their pointers name their address space (sa_common.h); through
+// generic ones every step of the panel update waited for the row operands
+// it had just asked for.  The FP64 kernel inlines everything.
+__device__ __noinline__ int nb_block_potrf(int w, sa_gf *D, long ldd, sa_gf *Dinv, sa_lf *S, sa_lf *Li)
 {
-	return block_potrf_inv64_t<T, true>(w, D, ldd, Dinv, S, Li);
+	return block_potrf_inv64_t<float, true>(w, (float *)D, ldd, (float *)Dinv, (float *)S, (float *)Li);
 }
 
-template <typename T>
-__device__ __noinline__ void nb_rows_apply(int rows, int w, const T *Dj, T *Pn, long ldp)
+__device__ __noinline__ void nb_rows_apply(int rows, int w, const sa_gf *Dj, sa_gf *Pn, long ldp)
 {
 	for (int row0 = (threadIdx.x >> 6) * 16; row0 < rows; row0 += 64)
-		rows_apply_inv_t<T>(row0, rows, w, Dj, Pn, ldp);
+		rows_apply_inv_t<float>(row0, rows, w, (const float *)Dj, (float *)Pn, ldp);
 }
 
-template <typename T, int RB>
-__device__ __noinline__ void nb_panel_update(int n, int j0, int w, T *A, T *Bs)
+__device__ __noinline__ void nb_panel_update(int n, int j0, int w, sa_gf *A, sa_lf *Bs)
 {
-	wg_panel_update<T, RB>(n, j0, w, A, Bs);
+	wg_panel_update<float, 2>(n, j0, w, (float *)A, (float *)Bs);
+}
+
+__device__ __noinline__ void nb_solve1(int n, const sa_gf *L, long ldl, const sa_gf *Dinv, sa_gf *x, sa_lf *Tl)
+{
+	wg_solve1<float>(n, (const float *)L, ldl, (const float *)Dinv, (float *)x, (float *)Tl);
 }
 
 // Left-looking factorisation of one n x n system (lower, ld n, in place)
@@ -324,7 +334,7 @@ __device__ __noinline__ void nb_panel_update(int n, int j0, int w, T *A, T *Bs)
 // inverse to the rows below; block inverses into Di.  Returns in thread 0
 // the 1-based column of the first non-positive pivot (or 0); *s_bad is LDS.
 template <typename T, int RB = 2>
-__device__ int wg_factor(int n, T *__restrict__ Ai, T *__restrict__ Di, T *__restrict__ S, T *__restrict__ Li,
+__device__ __forceinline__ int wg_factor(int n, T *__restrict__ Ai, T *__restrict__ Di, T *__restrict__ S, T *__restrict__ Li,
                          int *s_bad)
 {
 	if (threadIdx.x == 0)
@@ -333,12 +343,15 @@ __device__ int wg_factor(int n, T *__restrict__ Ai, T *__restrict__ Di, T *__res
 		const int w = (n - j0) < 64 ? (n - j0) : 64;
 		T *Dj = Di + 4096L * (j0 / 64);
 		if (j0 > 0) {
-			nb_panel_update<T, RB>(n, j0, w, Ai, S);
+			if constexpr (sizeof(T) == 4)
+				nb_panel_update(n, j0, w, (sa_gf *)Ai, (sa_lf *)S);
+			else
+				wg_panel_update<T, RB>(n, j0, w, Ai, S);
 			__syncthreads();
 		}
 		int bad;
 		if constexpr (sizeof(T) == 4)
-			bad = nb_block_potrf<T>(w, Ai + j0 + (long)j0 * n, n, Dj, S, Li);
+			bad = nb_block_potrf(w, (sa_gf *)(Ai + j0 + (long)j0 * n), n, (sa_gf *)Dj, (sa_lf *)S, (sa_lf *)Li);
 		else
 			bad = block_potrf_inv64_t<T, true>(w, Ai + j0 + (long)j0 * n, n, Dj, S, Li);
 		if (threadIdx.x == 0 && bad && bad <= w && *s_bad == 0)
@@ -347,7 +360,7 @@ __device__ int wg_factor(int n, T *__restrict__ Ai, T *__restrict__ Di, T *__res
 		if (rows > 0) {
 			T *Pn = Ai + (j0 + w) + (long)j0 * n;
 			if constexpr (sizeof(T) == 4)
-				nb_rows_apply<T>(rows, w, Dj, Pn, n);
+				nb_rows_apply(rows, w, (sa_gf *)Dj, (sa_gf *)Pn, n);
 			else
 				for (int row0 = (threadIdx.x >> 6) * 16; row0 < rows; row0 += 64)
 					rows_apply_inv_t<T>(row0, rows, w, Dj, Pn, n);
@@ -375,10 +388,9 @@ __device__ double wg_sum(double v, double *red4)
 // rows r0 + 64 m + l (m < NS); wave v walks the chunk's columns j = v,
 // v + 4, ..., NC of them per step.  NS * NC = 32 loads are in flight per
 // lane whatever the chunk's height.
-template <int NS, int NC>
-__device__ __noinline__ void residual_chunk(int r0, int r1, const double *__restrict__ A, long lda,
-                                               const double *__restrict__ x, double *__restrict__ r,
-                                               double *red)
+template <int NS, int NC, typename XD>
+__device__ __noinline__ void residual_chunk(int r0, int r1, const sa_gd *A, long lda, const XD *x, XD *r,
+                                            sa_ld *red)
 {
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	double acc[NS], xr[NS];
@@ -396,7 +408,7 @@ __device__ __noinline__ void residual_chunk(int r0, int r1, const double *__rest
 			const int jj = j + 4 * u;
 			const bool valid = jj < r1;
 			const double xj = valid ? x[jj] : 0.0;
-			const double *Aj = A + (long)(valid ? jj : 0) * lda;
+			const sa_gd *Aj = A + (long)(valid ? jj : 0) * lda;
 			const int mlo = jj > r0 ? (jj - r0) / 64 : 0;   // slots wholly above the diagonal
 			dot[u] = 0.0;
 			// loads independent of the lanes' masks (rows clamped into the
@@ -448,9 +460,9 @@ __device__ __noinline__ void residual_chunk(int r0, int r1, const double *__rest
 // product reduced over the wave into r_j (the upper product, A(j,i) =
 // A(i,j)).  The row accumulators of the four waves meet in `red` (4 * 1024
 // doubles of LDS).  Short chunks take more columns per step.
-__device__ __noinline__ double wg_residual(int n, const double *__restrict__ A, long lda, const double *__restrict__ b,
-                                          const double *__restrict__ x, double *__restrict__ r, double *red,
-                                          double *red4)
+template <typename XD>
+__device__ __forceinline__ double wg_residual(int n, const sa_gd *A, long lda, const sa_gd *b, const XD *x, XD *r,
+                                              sa_ld *red, double *red4)
 {
 	const int tid = threadIdx.x;
 	for (int i = tid; i < n; i += 256)
@@ -460,11 +472,11 @@ __device__ __noinline__ double wg_residual(int n, const double *__restrict__ A, 
 		const int r1 = (n - r0) < 1024 ? n : r0 + 1024;
 		const int h = r1 - r0;
 		if (h <= 256)
-			residual_chunk<4, 8>(r0, r1, A, lda, x, r, red);
+			residual_chunk<4, 8, XD>(r0, r1, A, lda, x, r, red);
 		else if (h <= 512)
-			residual_chunk<8, 4>(r0, r1, A, lda, x, r, red);
+			residual_chunk<8, 4, XD>(r0, r1, A, lda, x, r, red);
 		else
-			residual_chunk<16, 2>(r0, r1, A, lda, x, r, red);
+			residual_chunk<16, 2, XD>(r0, r1, A, lda, x, r, red);
 	}
 	double ss = 0.0;
 	for (int i = tid; i < n; i += 256)
@@ -512,7 +524,7 @@ void k_batched_potrs(int nsys, const int *__restrict__ order, const int *__restr
 // 64-row chunks (32 loads in flight per lane; only the lower triangle is
 // read).  Returns this thread's share of ||A||_F^2 (off-diagonal entries
 // twice).
-__device__ __noinline__ double wg_lower_to_f32(int n, const double *__restrict__ Ai, float *__restrict__ Afi)
+__device__ __noinline__ double wg_lower_to_f32(int n, const sa_gd *Ai, sa_gf *Afi)
 {
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	double ss = 0.0;
@@ -573,7 +585,7 @@ void k_batched_posv_ir(int nsys, const int *__restrict__ order, const int *__res
 	__shared__ double red4[4];
 	__shared__ int s_idx, s_bad;
 	float *S = SL, *Li = SL + 64 * LD;
-	double *red = reinterpret_cast<double *>(SL);
+	sa_ld *red = (sa_ld *)reinterpret_cast<double *>(SL);
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	for (;;) {
 		if (tid == 0)
@@ -588,20 +600,16 @@ void k_batched_posv_ir(int nsys, const int *__restrict__ order, const int *__res
 		const double *Ai = A + offA[sys];
 		float *Afi = Af + offA[sys];
 		float *Di = Dinvf + offD[sys];
-		const double ss = wg_lower_to_f32(n, Ai, Afi);
+		const double ss = wg_lower_to_f32(n, (const sa_gd *)Ai, (sa_gf *)Afi);
 		const double anorm = sqrt(wg_sum(ss, red4));
 		const int bad = wg_factor<float>(n, Afi, Di, S, Li, &s_bad);
 		for (int c = 0; c < nrhs; c++) {
 			const long o = offB[sys] + (long)c * n;
 			const double *b = B + o;
-			// x and r in LDS up to n = 1024 (the residual updates r column by
-			// column; in global memory each update was a dependent round trip)
-			const bool inl = n <= 1024;
-			double *x = inl ? xl : X + o, *r = inl ? rl : R + o;
 			float *d = Df + o;
 			int it = 0;
 			double be = __builtin_inf();
-			if (bad == 0) {
+			auto refine = [&](auto *x, auto *r) {
 				double bb = 0.0;
 				for (int i = tid; i < n; i += 256) {
 					const double v = b[i];
@@ -614,7 +622,7 @@ void k_batched_posv_ir(int nsys, const int *__restrict__ order, const int *__res
 					for (int i = tid; i < n; i += 256)
 						d[i] = (float)r[i];
 					__syncthreads();
-					wg_solve1<float>(n, Afi, n, Di, d, Tf);
+					nb_solve1(n, (const sa_gf *)Afi, n, (const sa_gf *)Di, (sa_gf *)d, (sa_lf *)Tf);
 					double xx = 0.0;
 					for (int i = tid; i < n; i += 256) {
 						const double v = x[i] + (double)d[i];
@@ -622,15 +630,23 @@ void k_batched_posv_ir(int nsys, const int *__restrict__ order, const int *__res
 						xx += v * v;
 					}
 					const double xnorm = sqrt(wg_sum(xx, red4));
-					const double rr = wg_residual(n, Ai, n, b, x, r, red, red4);
+					const double rr = wg_residual(n, (const sa_gd *)Ai, n, (const sa_gd *)b, x, r, red, red4);
 					it++;
 					be = rr == 0.0 ? 0.0 : sqrt(rr) / (anorm * xnorm + bnorm);
 					if (be <= tol)
 						break;
 				}
-				if (inl)
+			};
+			if (bad == 0) {
+				// x and r in LDS up to n = 1024 (the residual updates r column by
+				// column; in global memory each update was a dependent round trip)
+				if (n <= 1024) {
+					refine((sa_ld *)xl, (sa_ld *)rl);
 					for (int i = tid; i < n; i += 256)
 						X[o + i] = xl[i];
+				} else {
+					refine((sa_gd *)(X + o), (sa_gd *)(R + o));
+				}
 				__syncthreads();
 			}
 			if (tid == 0) {

@@ -472,7 +472,7 @@ __device__ __forceinline__ void store_inv64(const T *__restrict__ Li, T *__restr
 // One 256-thread workgroup; S, Li and the result as block_core64.  Ends with
 // a workgroup barrier, so the caller may reuse S and Li.
 template <typename T, bool FACTOR>
-__device__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__restrict__ Dinv, T *__restrict__ S,
+__device__ __forceinline__ int block_potrf_inv64_t(int w, T *__restrict__ D, long ldd, T *__restrict__ Dinv, T *__restrict__ S,
                                    T *__restrict__ Li)
 {
 	block_load64<T>(w, D, ldd, S, Li);

@@ -10,6 +10,15 @@ typedef double sa_d2 __attribute__((ext_vector_type(2)));
 typedef double sa_d4 __attribute__((ext_vector_type(4)));
 typedef float sa_f4 __attribute__((ext_vector_type(4)));
 
+// Pointers to device memory (g) and to LDS (l), for functions that are not
+// inlined and structs handed to them: through a generic pointer every load
+// is a FLAT access, which every wait for LDS data waits for as well.
+typedef __attribute__((address_space(1))) double sa_gd;
+typedef __attribute__((address_space(1))) float sa_gf;
+typedef __attribute__((address_space(1))) unsigned sa_gu;
+typedef __attribute__((address_space(3))) double sa_ld;
+typedef __attribute__((address_space(3))) float sa_lf;
+
 // v_mfma_f64_16x16x4f64: lane l supplies A(l%16, l/16) and B(l/16, l%16) of
 // a 16x4 by 4x16 product and accumulates D(4q + l/16, l%16) in register q.
 __device__ __forceinline__ sa_d4 sa_mfma(double a, double b, sa_d4 c)

@@ -107,27 +107,27 @@ struct PfArgs {
 	int factor;         // 1: factor A in place; 0: A holds the factor already
 	int inv;            // form W = L^-T (and Linv = L^-1 when Linv is given)
 	int delay;          // steps the inverse items trail the factor items by
-	double *A;
+	sa_gd *A;
 	long lda;
-	double *W;
+	sa_gd *W;
 	long ldw;
-	double *Linv;
+	sa_gd *Linv;
 	long ldi;
-	double *Dinv;       // nb blocks of 64x64 (ld 64)
-	unsigned *flags;
+	sa_gd *Dinv;      // nb blocks of 64x64 (ld 64)
+	sa_gu *flags;
 	int *info;
-	__device__ unsigned *rowl(int i) const { return flags + FLAG_STRIDE * i; }          // L(i,t) final for t < value
-	__device__ unsigned *diag(int i) const { return flags + FLAG_STRIDE * (nb + i); }   // A(i,i) but for t = i - 1
-	__device__ unsigned *sub(int i) const { return flags + FLAG_STRIDE * (2 * nb + i); } // A(i+1,i), all t < i
-	__device__ unsigned *dfin(int i) const { return flags + FLAG_STRIDE * (3 * nb + i); }
-	__device__ unsigned *roww(int j) const { return flags + FLAG_STRIDE * (4 * nb + j); } // W(j,t) final for t < value
-	__device__ unsigned *ticket() const { return flags + FLAG_STRIDE * (5 * nb); }
-	__device__ unsigned *abortf() const { return flags + FLAG_STRIDE * (5 * nb + 1); }
+	__device__ sa_gu *rowl(int i) const { return flags + FLAG_STRIDE * i; }          // L(i,t) final for t < value
+	__device__ sa_gu *diag(int i) const { return flags + FLAG_STRIDE * (nb + i); }   // A(i,i) but for t = i - 1
+	__device__ sa_gu *sub(int i) const { return flags + FLAG_STRIDE * (2 * nb + i); } // A(i+1,i), all t < i
+	__device__ sa_gu *dfin(int i) const { return flags + FLAG_STRIDE * (3 * nb + i); }
+	__device__ sa_gu *roww(int j) const { return flags + FLAG_STRIDE * (4 * nb + j); } // W(j,t) final for t < value
+	__device__ sa_gu *ticket() const { return flags + FLAG_STRIDE * (5 * nb); }
+	__device__ sa_gu *abortf() const { return flags + FLAG_STRIDE * (5 * nb + 1); }
 };
 
 __device__ __forceinline__ int bw(const PfArgs &p, int b) { return (p.n - 64 * b) < 64 ? (p.n - 64 * b) : 64; }
 
-__device__ __forceinline__ unsigned flag_read(const unsigned *f)
+__device__ __forceinline__ unsigned flag_read(const sa_gu *f)
 {
 	return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -141,7 +141,7 @@ constexpr unsigned SPIN_LIMIT = 1u << 22;
 // One wave waits until both counters have reached v (or the run is
 // abandoned) and then sees the data published before they were raised.
 // Returns the smaller counter, at least v.
-__device__ __forceinline__ int await(const PfArgs &p, const unsigned *f1, const unsigned *f2, int v)
+__device__ __forceinline__ int await(const PfArgs &p, const sa_gu *f1, const sa_gu *f2, int v)
 {
 	unsigned it = 0;
 	int m;
@@ -165,7 +165,7 @@ __device__ __forceinline__ int await(const PfArgs &p, const unsigned *f1, const 
 // raised.  Each wave waits for its own stores to complete before the
 // barrier; thread 0's agent-scope release then covers them all, so the L2
 // write-back runs once per item rather than once per wave.
-__device__ __forceinline__ void publish(unsigned *f, unsigned v)
+__device__ __forceinline__ void publish(sa_gu *f, unsigned v)
 {
 	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
 	__builtin_amdgcn_s_waitcnt(0);
@@ -185,11 +185,11 @@ __device__ __forceinline__ void publish(unsigned *f, unsigned v)
 // MFMAs; while a block's first half is multiplied the counters are read
 // again, so that a run goes on without a pause when more has become ready.
 struct Operand {
-	const double *p[2];     // the lane's two rows, column g
+	const sa_gd *p[2];      // the lane's two rows, column g
 	long ld;
 };
 
-__device__ __forceinline__ Operand operand(const double *X, long ld, int row0, int last)
+__device__ __forceinline__ Operand operand(const sa_gd *X, long ld, int row0, int last)
 {
 	const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	Operand o;
@@ -223,7 +223,7 @@ __device__ __forceinline__ void mul_half(const double (&xr)[2][8], const double 
 }
 
 __device__ __forceinline__ void accumulate(const PfArgs &p, const Operand &Pr, const Operand &Pc,
-                                           const unsigned *fr, const unsigned *fc, int t0, int t1,
+                                           const sa_gu *fr, const sa_gu *fc, int t0, int t1,
                                            sa_d4 (&acc)[2][2])
 {
 	double r0[2][8], c0[2][8], r1[2][8], c1[2][8];
@@ -269,7 +269,7 @@ __device__ __forceinline__ void accumulate(const PfArgs &p, const Operand &Pr, c
 // X = T inv^T for the wave's 16 rows 16 wave ..: T (64x64) in LDS, inv a
 // lower 64x64 block with leading dimension ldd (its zeros above the diagonal
 // are not multiplied).  x[cb][q] = X(16 wave + r, 16 cb + 4q + g).
-__device__ __forceinline__ void apply_inv(const double *T, const double *Dj, long ldd, sa_d4 (&x)[4])
+__device__ __forceinline__ void apply_inv(const double *T, const sa_gd *Dj, long ldd, sa_d4 (&x)[4])
 {
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	double dv[40];
@@ -300,7 +300,7 @@ __device__ __noinline__ void item_prepare(const PfArgs &p, int j, int l)
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
 	const int i = j + 1, wr = bw(p, i), wc = bw(p, l);
-	double *C = p.A + 64 * i + 64L * l * p.lda;
+	sa_gd *C = p.A + 64 * i + 64L * l * p.lda;
 	double cv[2][4][2];
 #pragma unroll
 	for (int bj = 0; bj < 2; bj++)
@@ -349,7 +349,7 @@ __device__ __noinline__ void item_P(const PfArgs &p, int i, int j, double *T)
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	const int i0 = 32 * (wave & 1), j0 = 32 * (wave >> 1);
 	const int wr = bw(p, i);            // block column j < i is full
-	double *C = p.A + 64 * i + 64L * j * p.lda;
+	sa_gd *C = p.A + 64 * i + 64L * j * p.lda;
 	double cv[2][4][2];
 #pragma unroll
 	for (int bj = 0; bj < 2; bj++)
@@ -380,7 +380,8 @@ __device__ __noinline__ void item_P(const PfArgs &p, int i, int j, double *T)
 // The inverse of diagonal block j of a tile that is factored already.
 __device__ __noinline__ void item_D(const PfArgs &p, int j, double *S, double *Li)
 {
-	block_potrf_inv64<false>(bw(p, j), p.A + 64 * j + 64L * j * p.lda, p.lda, p.Dinv + 4096L * j, S, Li);
+	block_potrf_inv64<false>(bw(p, j), (double *)(p.A + 64 * j + 64L * j * p.lda), p.lda, (double *)(p.Dinv + 4096L * j), S,
+	                         Li);
 	publish(p.dfin(j), 1u);
 }
 
@@ -392,8 +393,8 @@ __device__ __noinline__ void item_WD(const PfArgs &p, int t)
 {
 	await(p, p.dfin(t), p.dfin(t), 1);
 	const int w = bw(p, t);
-	const double *D = p.Dinv + 4096L * t;
-	double *Wb = p.W + 64 * t + 64L * t * p.ldw;
+	const sa_gd *D = p.Dinv + 4096L * t;
+	sa_gd *Wb = p.W + 64 * t + 64L * t * p.ldw;
 	double u[16], v[16];
 #pragma unroll
 	for (int q = 0; q < 16; q++) {
@@ -430,7 +431,7 @@ __device__ __noinline__ void item_WX(const PfArgs &p, int j, int i, double *T, d
 	sa_d4 x[4];
 	apply_inv(T, p.Dinv + 4096L * i, 64, x);
 	const int row = 16 * wave + r;
-	double *Wb = p.W + 64 * j + 64L * i * p.ldw;
+	sa_gd *Wb = p.W + 64 * j + 64L * i * p.ldw;
 #pragma unroll
 	for (int cb = 0; cb < 4; cb++)
 #pragma unroll
@@ -461,25 +462,25 @@ __device__ __noinline__ void item_WX(const PfArgs &p, int j, int i, double *T, d
 // and inverted in LDS and its inverse published; L(j+1,j) is formed from the
 // prepared A(j+1,j) and the inverse in LDS, published, and kept in LDS for
 // the last update of A(j+1,j+1), which becomes the next S.
-__device__ void run_chain(const PfArgs &p, double *S, double *Li)
+__device__ __forceinline__ void run_chain(const PfArgs &p, double *S, double *Li)
 {
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
 	int first_bad = 0;
 	if (p.nb > 0)
-		block_load64<double>(bw(p, 0), p.A, p.lda, S, Li);
+		block_load64<double>(bw(p, 0), (double *)p.A, p.lda, S, Li);
 	for (int j = 0; j < p.nb; j++) {
 		const int wj = bw(p, j);
 		const int bad = block_core64<double, true>(S, Li);
 		if (threadIdx.x == 0 && bad && bad <= wj && first_bad == 0)
 			first_bad = 64 * j + bad;
-		store_inv64<double>(Li, p.Dinv + 4096L * j);
-		store_lower64<double>(wj, S, p.A + 64 * j + 64L * j * p.lda, p.lda);
+		store_inv64<double>(Li, (double *)(p.Dinv + 4096L * j));
+		store_lower64<double>(wj, S, (double *)(p.A + 64 * j + 64L * j * p.lda), p.lda);
 		if (j + 1 == p.nb) {
 			publish(p.dfin(j), 1u);
 			break;
 		}
 		const int wn = bw(p, j + 1);
-		double *P = p.A + 64 * (j + 1) + 64L * j * p.lda, *C = p.A + 64 * (j + 1) + 64L * (j + 1) * p.lda;
+		sa_gd *P = p.A + 64 * (j + 1) + 64L * j * p.lda, *C = p.A + 64 * (j + 1) + 64L * (j + 1) * p.lda;
 		// the wave's 16 rows of A(j+1,j), and its blocks of the lower half of
 		// A(j+1,j+1): 16x16 blocks 4u + wave of the ten, row by row
 		const int row = 16 * wave + r, rowc = row < wn ? row : wn - 1;
@@ -625,7 +626,7 @@ __host__ __device__ inline Cursor cursor_first(const PfOrder &o, bool *valid)
 // and every item waits only for items earlier in the order, so the earliest
 // unfinished item is always held by a running workgroup with its inputs
 // ready; an item not yet handed out blocks nobody.
-__device__ void run_bulk(const PfArgs &p, double *S, double *Li, int *s_ticket)
+__device__ __forceinline__ void run_bulk(const PfArgs &p, double *S, double *Li, int *s_ticket)
 {
 	const PfOrder o = {p.nb, p.factor, p.inv, p.delay};
 	bool valid;
@@ -634,7 +635,7 @@ __device__ void run_bulk(const PfArgs &p, double *S, double *Li, int *s_ticket)
 	for (;;) {
 		__syncthreads();                  // the last item's reads of LDS are done
 		if (threadIdx.x == 0)
-			*s_ticket = (int)atomicAdd(p.ticket(), 1u);
+			*s_ticket = (int)__hip_atomic_fetch_add(p.ticket(), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		__syncthreads();
 		const int t = *s_ticket;
 		while (valid && pos < t) {
@@ -733,21 +734,21 @@ int launch_tile(hipStream_t s, int n, double *A, int lda, int *dev_info, void *w
 	p.factor = factor;
 	p.inv = W != nullptr;
 	p.delay = factor ? 1 : 0;
-	p.A = A;
+	p.A = (sa_gd *)A;
 	p.lda = lda;
-	p.W = W;
+	p.W = (sa_gd *)W;
 	p.ldw = ldw;
-	p.Linv = Linv;
+	p.Linv = (sa_gd *)Linv;
 	p.ldi = ldi;
-	p.Dinv = (double *)ws;
-	p.flags = (unsigned *)(ws + align256((size_t)(nb ? nb : 1) * 4096 * sizeof(double)));
+	p.Dinv = (sa_gd *)ws;
+	p.flags = (sa_gu *)(ws + align256((size_t)(nb ? nb : 1) * 4096 * sizeof(double)));
 	p.info = dev_info;
 	if (nb == 0) {
 		if (!factor)
 			return 0;
 		// n = 0: reports info = 0
 		p.nbulk = 0;
-		hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(64), 0, s, p.flags, 1, 1);
+		hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(64), 0, s, (unsigned *)p.flags, 1, 1);
 		int e = sa_launch_status();
 		if (e)
 			return e;
@@ -757,7 +758,7 @@ int launch_tile(hipStream_t s, int n, double *A, int lda, int *dev_info, void *w
 	const long items = count_items(PfOrder{nb, factor, p.inv, p.delay});
 	const int want = bulk > 0 ? (bulk < 255 ? bulk : 255) : max_bulk();
 	p.nbulk = (int)(items < want ? items : want);
-	hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(256), 0, s, p.flags, nb, factor);
+	hipLaunchKernelGGL(k_init_counters, dim3(1), dim3(256), 0, s, (unsigned *)p.flags, nb, factor);
 	int e = sa_launch_status();
 	if (e)
 		return e;
