@@ -73,6 +73,8 @@ template <> struct StageT<MODE_F32> { typedef float type; static constexpr int p
 
 typedef float sa_f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef __bf16 sa_bf4 __attribute__((ext_vector_type(4)));
+typedef __bf16 sa_bf2 __attribute__((ext_vector_type(2)));
+typedef float sa_f2 __attribute__((ext_vector_type(2)));
 
 template <int MODE, int WB, bool UPPER>
 __global__ __launch_bounds__(256)
@@ -138,12 +140,23 @@ void k_sgemm_lds(int M, int N, int K, float alpha, const float *__restrict__ A, 
 		if constexpr (MODE == MODE_F32) {
 			*reinterpret_cast<sa_f4 *>(p) = x;
 		} else {
+			// two values per conversion; a bf16 is the upper half of its FP32
+			// form, so hi is taken back from the packed pair, not converted
 			sa_bf4 h, l;
 #pragma unroll
-			for (int e = 0; e < 4; e++) {
-				h[e] = (__bf16)x[e];
-				if (NPL == 2)
-					l[e] = (__bf16)(x[e] - (float)h[e]);
+			for (int e = 0; e < 4; e += 2) {
+				const sa_f2 v = {x[e], x[e + 1]};
+				const sa_bf2 hv = __builtin_convertvector(v, sa_bf2);
+				h[e] = hv[0];
+				h[e + 1] = hv[1];
+				if (NPL == 2) {
+					const unsigned u = __builtin_bit_cast(unsigned, hv);
+					const sa_f2 d = {v[0] - __builtin_bit_cast(float, u << 16),
+					                 v[1] - __builtin_bit_cast(float, u & 0xffff0000u)};
+					const sa_bf2 lv = __builtin_convertvector(d, sa_bf2);
+					l[e] = lv[0];
+					l[e + 1] = lv[1];
+				}
 			}
 			*reinterpret_cast<sa_bf4 *>(p) = h;
 			if (NPL == 2)
@@ -214,7 +227,7 @@ void k_sgemm_lds(int M, int N, int K, float alpha, const float *__restrict__ A, 
 		constexpr int NM = WB * WB * (MODE == MODE_F32 ? 8 : MODE == MODE_BF16X3 ? 3 : 1);   // MFMAs
 		constexpr int NR = 2 * WB * (MODE == MODE_BF16 ? 1 : 2);                             // LDS reads
 		constexpr int NS = 2 * WB * NPL, NG = 2 * WB;                                        // LDS stores, loads
-		constexpr int NV = MODE == MODE_F32 ? 0 : 2 * WB * (NPL == 2 ? 14 : 4);              // conversions, about
+		constexpr int NV = MODE == MODE_F32 ? 0 : 2 * WB * (NPL == 2 ? 12 : 2);              // conversions, about
 		constexpr int H = NM / 3 > 0 ? NM / 3 : 1;
 #pragma unroll
 		for (int q = 0; q < NM; q++) {
@@ -629,17 +642,19 @@ void k_split_bf16x2(int m, int n, const float *__restrict__ A, long lda, __bf16 
 	L[i + (long)j * ldh] = (__bf16)(x - (float)h);
 }
 
-// 64x64 workgroup tiles up to products that give 192 workgroups of 128x128:
-// four times the workgroups, three on a compute unit (against one of
-// 128x128), which alone and with four launches in flight is the faster:
-// 1024^3 FP32 23.1 / 20.8 us against 67.9 / 35.0, BF16x3 18.3 / 13.9 against
-// 31.7 / 17.5.
+// 64x64 workgroup tiles up to products that give 192 workgroups of 128x128
+// (FP32) or 64 (BF16 forms): four times the workgroups, three on a compute
+// unit against one.  Alone, 1024^3 FP32 takes 23.1 us against 67.9 and with
+// four launches in flight 20.8 against 35.0; BF16x3, where the 64x64 form
+// spends its time on LDS reads, 18.3 against 31.7 alone, but the N=32768
+// factorisation on 1024 tiles with four hardware queues runs its 128x128
+// form in 90.7 ms (solve included) against 95.5, 512 tiles the 64x64 form.
 template <int MODE, bool UPPER>
 int sgemm_shape(hipStream_t s, int m, int n, int k, float alpha, const float *A, int lda, const float *B,
                 int ldb, float beta, float *C, int ldc, int ktri = 0)
 {
 	const long tm = (m + 127) / 128, tn = (n + 127) / 128;
-	if ((UPPER ? tn * (tn + 1) / 2 : tm * tn) >= 192)
+	if ((UPPER ? tn * (tn + 1) / 2 : tm * tn) >= (MODE == MODE_F32 ? 192 : 64))
 		return sgemm_lds<MODE, 4, UPPER>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
 	return sgemm_lds<MODE, 2, UPPER>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, ktri);
 }
