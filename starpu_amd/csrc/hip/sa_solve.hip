@@ -405,33 +405,35 @@ void k_gemm_thin_mfma(int m, int r, int kdim, int kc, double alpha, const TA *__
 		}
 }
 
-// Thin product for the solves with an FP32 factor, C(m x r) = beta*C +
-// alpha*op(A)*B with A FP32 and B, C FP64, without partial sums in memory:
-// a workgroup computes 16 RB rows x 16 right-hand sides (rows 16 RB x..,
-// columns 16y..), its NW waves each take a contiguous share of k (whole
-// 32-wide steps) and all RB 16-row blocks, with the lane layout of
-// k_gemm_thin_mfma -- lane l supplies k = k0 + 8g + b at MFMA step b
-// (g = l/16), B's element for column l%16 and A's for row l%16 of each
-// block -- and the waves' partial sums meet in LDS, added in wave order, so
-// the result never depends on timing.  A wave issues the loads of U steps
-// before their MFMAs: the product is bound by load latency, and one round
-// trip per U steps replaces one per step.  The RB blocks of a wave share its
-// B values: with RB = 1 (short products, 16-row workgroups: a 1024-row
-// product gets 64 of them) every workgroup reads all of its k-range of B
-// per 16 rows, which on tall operands moves twice the bytes of A through
-// the caches and ran a 31744 x 1024 panel at 2 TB/s; RB = 4 shares each B
-// load among four blocks.  TN reads 8 consecutive k of A's column as two
-// 4-float vectors (host: k % 8 == 0, lda % 4 == 0, A 16-byte aligned); NN
-// reads A(row, k) per k, for RB = 4 as one 4-row vector per k with block j
-// holding rows 16 RB x + 4i + j (host: also m % 4 == 0).
-template <bool TRANS, int RB, int NW>
+// Thin product without partial sums in memory, one launch: C(m x r) = beta*C
+// + alpha*op(A)*B with A FP32 or FP64 and B, C FP64.  A workgroup computes
+// 16 RB rows x 16 right-hand sides (rows 16 RB x.., columns 16y..), its NW
+// waves each take a contiguous share of k (whole 32-wide steps) and all RB
+// 16-row blocks, with the lane layout of k_gemm_thin_mfma -- lane l supplies
+// k = k0 + 8g + b at MFMA step b (g = l/16), B's element for column l%16 and
+// A's for row l%16 of each block -- and the waves' partial sums meet in LDS,
+// added in wave order, so the result never depends on timing.  A wave issues
+// the loads of U steps before their MFMAs: the product is bound by load
+// latency, and one round trip per U steps replaces one per step.  The RB
+// blocks of a wave share its B values: with RB = 1 (short products, 16-row
+// workgroups: a 1024-row product gets 64 of them) every workgroup reads all
+// of its k-range of B per 16 rows, which on tall operands moves twice the
+// bytes of A through the caches and ran a 31744 x 1024 FP32 panel at 2 TB/s;
+// RB = 4 shares each B load among four blocks.  TN reads 8 consecutive k of
+// A's column as two 4-element vectors; NN reads A(row, k) per k, for RB = 4 as
+// one 4-row vector per k with block j holding rows 16 RB x + 4i + j (host:
+// m % 4 == 0).  The vectors need only the alignment of an element, and the
+// last kdim % 32 columns go element by element, so any k, leading dimension
+// and offset takes this form.
+template <bool TRANS, int RB, int NW, typename TA>
 __global__ __launch_bounds__(64 * NW)
-void k_thin_rows(int m, int r, int kdim, double alpha, const float *__restrict__ A, long lda,
+void k_thin_rows(int m, int r, int kdim, double alpha, const TA *__restrict__ A, long lda,
                  const double *__restrict__ B, long ldb, double beta, double *__restrict__ C, long ldc)
 {
-	typedef float TA4 __attribute__((ext_vector_type(4)));
+	typedef TA TA4 __attribute__((ext_vector_type(4), aligned(sizeof(TA))));
+	typedef double D2 __attribute__((ext_vector_type(2), aligned(8)));
 	static_assert(RB == 1 || RB == 4, "row blocks per wave: 1 or 4");
-	constexpr int U = RB == 1 ? 4 : 2;
+	constexpr int U = RB == 1 ? 4 : sizeof(TA) == 4 ? 2 : 1;
 	__shared__ sa_d4 part[NW - 1][RB][64];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int l16 = lane & 15, g = lane >> 4;
@@ -442,28 +444,35 @@ void k_thin_rows(int m, int r, int kdim, double alpha, const float *__restrict__
 	const int steps = (kdim + 31) / 32, per = (steps + NW - 1) / NW;
 	const int sb = wave * per;
 	const int se = (steps - sb) < per ? steps : sb + per;
+	const int sf = se < kdim / 32 ? se : kdim / 32;      // whole steps of this wave
+	const TA *pa[RB];
+#pragma unroll
+	for (int j = 0; j < RB; j++) {
+		const int row = TRANS || RB == 1 ? row0 + 16 * j + l16 : row0 + 4 * l16;
+		const int rc = row < m ? row : TRANS || RB == 1 ? m - 1 : 0;
+		pa[j] = TRANS ? A + (long)rc * lda : A + rc;
+	}
 	sa_d4 acc[RB];
 #pragma unroll
 	for (int j = 0; j < RB; j++)
 		acc[j] = sa_d4{0.0, 0.0, 0.0, 0.0};
-	for (int s0 = sb; s0 < se; s0 += U) {
-		float av[U][RB][8];
+	for (int s0 = sb; s0 < sf; s0 += U) {
+		TA av[U][RB][8];
 		double bv[U][8];
-		bool kin[U];
 #pragma unroll
 		for (int u = 0; u < U; u++) {
-			const int kk = 32 * (s0 + u) + 8 * g;
-			kin[u] = s0 + u < se && kk < kdim;
-			const int kl = kin[u] ? kk : 32 * sb;
+			const int kl = 32 * (s0 + u < sf ? s0 + u : sb) + 8 * g;
 #pragma unroll
-			for (int b = 0; b < 8; b++)
-				bv[u][b] = Bc[kl + b];
+			for (int b = 0; b < 8; b += 2) {
+				const D2 x = *reinterpret_cast<const D2 *>(Bc + kl + b);
+				bv[u][b] = x.x;
+				bv[u][b + 1] = x.y;
+			}
 			if (TRANS) {
 #pragma unroll
 				for (int j = 0; j < RB; j++) {
-					const int row = row0 + 16 * j + l16;
-					const float *pa = A + kl + (long)(row < m ? row : m - 1) * lda;
-					const TA4 x0 = *reinterpret_cast<const TA4 *>(pa), x1 = *reinterpret_cast<const TA4 *>(pa + 4);
+					const TA4 x0 = *reinterpret_cast<const TA4 *>(pa[j] + kl);
+					const TA4 x1 = *reinterpret_cast<const TA4 *>(pa[j] + kl + 4);
 #pragma unroll
 					for (int e = 0; e < 4; e++) {
 						av[u][j][e] = x0[e];
@@ -471,17 +480,13 @@ void k_thin_rows(int m, int r, int kdim, double alpha, const float *__restrict__
 					}
 				}
 			} else if (RB == 1) {
-				const int row = row0 + l16;
-				const int rowc = row < m ? row : m - 1;
 #pragma unroll
 				for (int b = 0; b < 8; b++)
-					av[u][0][b] = A[rowc + (long)(kl + b) * lda];
+					av[u][0][b] = pa[0][(long)(kl + b) * lda];
 			} else {
-				const int rw = row0 + 4 * l16;
-				const float *pa = A + (rw < m ? rw : 0);
 #pragma unroll
 				for (int b = 0; b < 8; b++) {
-					const TA4 x = *reinterpret_cast<const TA4 *>(pa + (long)(kl + b) * lda);
+					const TA4 x = *reinterpret_cast<const TA4 *>(pa[0] + (long)(kl + b) * lda);
 #pragma unroll
 					for (int j = 0; j < RB; j++)
 						av[u][j][b] = x[j];
@@ -489,13 +494,30 @@ void k_thin_rows(int m, int r, int kdim, double alpha, const float *__restrict__
 			}
 		}
 #pragma unroll
-		for (int u = 0; u < U; u++)
+		for (int u = 0; u < U; u++) {
+			const bool on = s0 + u < sf;
 #pragma unroll
 			for (int b = 0; b < 8; b++)
 #pragma unroll
 				for (int j = 0; j < RB; j++)
-					acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(kin[u] ? (double)av[u][j][b] : 0.0,
-					                                               (kin[u] && cin) ? bv[u][b] : 0.0, acc[j], 0, 0, 0);
+					acc[j] = sa_mfma(on ? (double)av[u][j][b] : 0.0, (on && cin) ? bv[u][b] : 0.0, acc[j]);
+		}
+	}
+	if (sb < se && sf < se) {
+		// the last kdim % 32 columns: the step after kdim / 32 whole ones, of
+		// the one wave whose share it ends
+#pragma unroll
+		for (int b = 0; b < 8; b++) {
+			const int k = 32 * sf + 8 * g + b, kc = k < kdim ? k : kdim - 1;
+			const bool on = k < kdim;
+			const double bw = Bc[kc];
+#pragma unroll
+			for (int j = 0; j < RB; j++) {
+				const double x = (double)(TRANS ? pa[j][kc] : RB == 1 ? pa[0][(long)kc * lda]
+				                                                     : pa[0][j + (long)kc * lda]);
+				acc[j] = sa_mfma(on ? x : 0.0, (on && cin) ? bw : 0.0, acc[j]);
+			}
+		}
 	}
 	if (wave > 0)
 #pragma unroll
@@ -522,7 +544,7 @@ void k_thin_rows(int m, int r, int kdim, double alpha, const float *__restrict__
 		}
 }
 
-// Shape of k_thin_rows for an m-row product: 16-row workgroups of eight
+// Shape of k_thin_rows for an m-row FP32 product: 16-row workgroups of eight
 // waves below thin_tall_min_m() rows, 64-row workgroups (four blocks per
 // wave) of thin_tall_waves() waves from there.  SA_THIN_TALL_MIN_M and
 // SA_THIN_TALL_WAVES (4 or 8) override, for tuning.
@@ -547,10 +569,10 @@ int thin_tall_waves()
 	return v;
 }
 
-// k_thin_rows when its layout conditions hold (SA_THIN_ROWS16=0 turns it
-// off); 1 if the caller should take the split-k forms.
-template <bool TRANS>
-int thin_rows16(hipStream_t s, int m, int r, int k, double alpha, const float *A, int lda, const double *B, int ldb,
+// k_thin_rows (SA_THIN_ROWS16=0 turns it off); 1 if the caller should take
+// the split-k forms.
+template <bool TRANS, typename TA>
+int thin_rows16(hipStream_t s, int m, int r, int k, double alpha, const TA *A, int lda, const double *B, int ldb,
                 double beta, double *C, int ldc, int *status)
 {
 	static int on = -1;
@@ -558,23 +580,24 @@ int thin_rows16(hipStream_t s, int m, int r, int k, double alpha, const float *A
 		const char *e = getenv("SA_THIN_ROWS16");
 		on = (e && atoi(e) == 0) ? 0 : 1;
 	}
-	if (!on || k % 8 != 0 || (TRANS && (lda % 4 != 0 || ((uintptr_t)A % 16) != 0)))
+	if (!on)
 		return 1;
-	const bool tall = m >= thin_tall_min_m() &&
-	                  (TRANS || (m % 4 == 0 && lda % 4 == 0 && ((uintptr_t)A % 16) == 0));
-	if (tall) {
-		const dim3 grid((unsigned)((m + 63) / 64), (unsigned)((r + 15) / 16));
-		if (thin_tall_waves() == 4)
-			hipLaunchKernelGGL((k_thin_rows<TRANS, 4, 4>), grid, dim3(256), 0, s, m, r, k, alpha, A, (long)lda, B,
-			                   (long)ldb, beta, C, (long)ldc);
-		else
-			hipLaunchKernelGGL((k_thin_rows<TRANS, 4, 8>), grid, dim3(512), 0, s, m, r, k, alpha, A, (long)lda, B,
-			                   (long)ldb, beta, C, (long)ldc);
-	} else {
-		const dim3 grid((unsigned)((m + 15) / 16), (unsigned)((r + 15) / 16));
-		hipLaunchKernelGGL((k_thin_rows<TRANS, 1, 8>), grid, dim3(512), 0, s, m, r, k, alpha, A, (long)lda, B,
-		                   (long)ldb, beta, C, (long)ldc);
+	if constexpr (sizeof(TA) == 4) {
+		if (m >= thin_tall_min_m() && (TRANS || m % 4 == 0)) {
+			const dim3 grid((unsigned)((m + 63) / 64), (unsigned)((r + 15) / 16));
+			if (thin_tall_waves() == 4)
+				hipLaunchKernelGGL((k_thin_rows<TRANS, 4, 4, TA>), grid, dim3(256), 0, s, m, r, k, alpha, A,
+				                   (long)lda, B, (long)ldb, beta, C, (long)ldc);
+			else
+				hipLaunchKernelGGL((k_thin_rows<TRANS, 4, 8, TA>), grid, dim3(512), 0, s, m, r, k, alpha, A,
+				                   (long)lda, B, (long)ldb, beta, C, (long)ldc);
+			*status = sa_launch_status();
+			return 0;
+		}
 	}
+	const dim3 grid((unsigned)((m + 15) / 16), (unsigned)((r + 15) / 16));
+	hipLaunchKernelGGL((k_thin_rows<TRANS, 1, 8, TA>), grid, dim3(512), 0, s, m, r, k, alpha, A, (long)lda, B,
+	                   (long)ldb, beta, C, (long)ldc);
 	*status = sa_launch_status();
 	return 0;
 }
@@ -716,6 +739,15 @@ int gemm_thin_mfma(hipStream_t s, int m, int r, int k, double alpha, const TA *A
 	return 0;
 }
 
+// FP64 products that take k_thin_rows (SA_THIN_ROWS16=0: none): the solves'
+// tile and panel products.  Beyond, the MFMA form split over k, which shares
+// B among more rows.  From memory, k = 1024, 16 right-hand sides (us, NN / TN,
+// against the forms split over k with their reduction): 1024 rows 17.0 / 16.5
+// and 22.0 / 20.2, 2048 rows 19.0 / 18.1 and 23.8 / 24.3, 4096 rows 21.7 /
+// 20.4 and 31.9 / 32.8, 8192 rows 36.6 / 34.8 and 38.9 / 40.9, 15360 rows
+// 64.2 / 62.1 and 58.6 / 61.6.
+constexpr int THIN_ROWS_MAX_K = 2048, THIN_ROWS_MAX_M = 12288;
+
 template <bool TRANS, typename TA = double>
 int gemm_thin(hipStream_t s, int m, int r, int k, double alpha, const TA *A, int lda,
               const double *B, int ldb, double beta, double *C, int ldc, void *work, size_t work_bytes)
@@ -725,6 +757,9 @@ int gemm_thin(hipStream_t s, int m, int r, int k, double alpha, const TA *A, int
 	if (k == 0)
 		return beta == 1.0 ? 0 : sa_scale_launch(s, m, r, C, ldc, beta, false);
 	int status = 0;
+	if (k <= THIN_ROWS_MAX_K && m <= THIN_ROWS_MAX_M &&
+	    thin_rows16<TRANS, TA>(s, m, r, k, alpha, A, lda, B, ldb, beta, C, ldc, &status) == 0)
+		return status;
 	if (gemm_thin_mfma<TRANS, TA>(s, m, r, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, &status) == 0)
 		return status;
 	constexpr int tk = thin_tk<TA>();
@@ -905,7 +940,7 @@ extern "C" int sa_gemm_nn_sd(hipStream_t s, int m, int n, int k, double alpha, c
 	if (m < 0 || n < 0 || k < 0 || !ld_ok(lda, m) || !ld_ok(ldb, k) || !ld_ok(ldc, m))
 		return -EINVAL;
 	int status = 0;
-	if (m > 0 && n > 0 && k > 0 && thin_rows16<false>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, &status) == 0)
+	if (m > 0 && n > 0 && k > 0 && thin_rows16<false, float>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, &status) == 0)
 		return status;
 	return gemm_thin<false, float>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes);
 }
@@ -917,7 +952,7 @@ extern "C" int sa_gemm_tn_sd(hipStream_t s, int m, int n, int k, double alpha, c
 	if (m < 0 || n < 0 || k < 0 || !ld_ok(lda, k) || !ld_ok(ldb, k) || !ld_ok(ldc, m))
 		return -EINVAL;
 	int status = 0;
-	if (m > 0 && n > 0 && k > 0 && thin_rows16<true>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, &status) == 0)
+	if (m > 0 && n > 0 && k > 0 && thin_rows16<true, float>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, &status) == 0)
 		return status;
 	return gemm_thin<true, float>(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes);
 }

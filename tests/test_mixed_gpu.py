@@ -274,6 +274,29 @@ def test_fp32_factor_solve_kernels(K, m, n, k):
         assert np.linalg.norm(dX.download() - exp) / np.linalg.norm(exp) < 1e-13
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("m,r", [(1, 1), (17, 16), (100, 17), (4097, 3), (4100, 16)])
+@pytest.mark.parametrize("k", [1, 7, 32, 33, 95, 255, 256, 257, 300])
+def test_thin_rows_k_shares(K, dtype, m, r, k):
+    # the one-launch thin product: k shares of the eight waves that are empty,
+    # whole and ragged, both row forms, columns aligned to an element only;
+    # integers, so a step taken twice or left out changes the exact result
+    print(f"thin rows {dtype.__name__} m={m} r={r} k={k}", flush=True)
+    L = K.lib()
+    rng = np.random.default_rng(m + 3 * r + 7 * k)
+    A, B = rng.integers(-9, 10, (m, k)).astype(dtype), rng.integers(-9, 10, (k, r)).astype(float)
+    C0 = rng.integers(-64, 65, (m + 1, r)).astype(float)
+    nn, tn = (L.sa_dgemm_nn, L.sa_dgemm_tn) if dtype is np.float64 else (L.sa_gemm_nn_sd, L.sa_gemm_tn_sd)
+    dN, dT = K.DeviceArray.from_host(A, ld=m + 1), K.DeviceArray.from_host(np.asfortranarray(A.T), ld=k + 1)
+    dB = K.DeviceArray.from_host(B, ld=k + 3)
+    exp = C0.copy()
+    exp[:m] = 2.0 * C0[:m] - A.astype(float) @ B
+    for f, dA in ((nn, dN), (tn, dT)):
+        dC = K.DeviceArray.from_host(C0)
+        K.check(f(None, m, r, k, -1.0, dA.ptr, dA.ld, dB.ptr, dB.ld, 2.0, dC.ptr, dC.ld, None, 0), "thin")
+        assert np.array_equal(dC.download(), exp)
+
+
 @pytest.mark.parametrize("n,r", [(1, 1), (17, 3), (255, 16), (256, 16), (300, 17), (1000, 5), (2049, 16),
                                  (4500, 16), (8192, 16)])
 def test_symmetric_residual_reads_lower_triangle_only(K, n, r):
