@@ -305,8 +305,8 @@ void k_thin_reduce(int m, int r, int ns, double alpha, const double *__restrict_
 	*p = (beta == 0.0 ? 0.0 : beta * cv) + alpha * s;
 }
 
-// MFMA form of the thin GEMM for tall operands (m >= 2048): FP64
-// MFMAs (v_mfma_f64_16x16x4f64) instead of FMAs on the VALU, whose
+// MFMA form of the thin GEMM for tall operands (m >= 2048) that k_thin_rows
+// does not take (FP64 with m > 12288 or k > 2048): FP64 MFMAs (v_mfma_f64_16x16x4f64) instead of FMAs on the VALU, whose
 // right-hand-side reads from LDS (16 doubles per k and lane) bounded
 // k_gemm_thin at ~1.5 TB/s on such shapes.  Workgroup (x, y, z): four waves
 // of 64 rows each (rows 256x + 64 wave ..), k slice y (kc columns of op(A)),
