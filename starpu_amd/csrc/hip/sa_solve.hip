@@ -306,7 +306,7 @@ void k_thin_reduce(int m, int r, int ns, double alpha, const double *__restrict_
 }
 
 // MFMA form of the thin GEMM for tall operands (m >= 2048) that k_thin_rows
-// does not take (FP64 with m > 12288 or k > 2048): FP64 MFMAs (v_mfma_f64_16x16x4f64) instead of FMAs on the VALU, whose
+// does not take (thin_rows_wins): FP64 MFMAs (v_mfma_f64_16x16x4f64) instead of FMAs on the VALU, whose
 // right-hand-side reads from LDS (16 doubles per k and lane) bounded
 // k_gemm_thin at ~1.5 TB/s on such shapes.  Workgroup (x, y, z): four waves
 // of 64 rows each (rows 256x + 64 wave ..), k slice y (kc columns of op(A)),
@@ -745,8 +745,18 @@ int gemm_thin_mfma(hipStream_t s, int m, int r, int k, double alpha, const TA *A
 // against the forms split over k with their reduction): 1024 rows 17.0 / 16.5
 // and 22.0 / 20.2, 2048 rows 19.0 / 18.1 and 23.8 / 24.3, 4096 rows 21.7 /
 // 20.4 and 31.9 / 32.8, 8192 rows 36.6 / 34.8 and 38.9 / 40.9, 15360 rows
-// 64.2 / 62.1 and 58.6 / 61.6.
+// 64.2 / 62.1 and 58.6 / 61.6.  A workgroup holds 16 right-hand sides, so a
+// group of 16 more costs as the same rows once more: 32 right-hand sides
+// 27.1 / 29.0 and 31.9 / 33.6 at 4096 rows, 49.4 / 51.3 and 42.1 / 49.4 at
+// 8192; 64 at 4096 rows 39.8 / 43.9 and 33.5 / 39.8.  Below the rows the MFMA
+// form takes, it wins whatever their number (1024 rows: 64 17.1 / 15.6 and
+// 32.4 / 34.5, 512 58 / 74 and 155 / 180).
 constexpr int THIN_ROWS_MAX_K = 2048, THIN_ROWS_MAX_M = 12288;
+
+bool thin_rows_wins(int m, int r, int k)
+{
+	return k <= THIN_ROWS_MAX_K && (m < MFMA_MIN_M || (long)m * ((r + 15) / 16) <= THIN_ROWS_MAX_M);
+}
 
 template <bool TRANS, typename TA = double>
 int gemm_thin(hipStream_t s, int m, int r, int k, double alpha, const TA *A, int lda,
@@ -757,7 +767,7 @@ int gemm_thin(hipStream_t s, int m, int r, int k, double alpha, const TA *A, int
 	if (k == 0)
 		return beta == 1.0 ? 0 : sa_scale_launch(s, m, r, C, ldc, beta, false);
 	int status = 0;
-	if (k <= THIN_ROWS_MAX_K && m <= THIN_ROWS_MAX_M &&
+	if (thin_rows_wins(m, r, k) &&
 	    thin_rows16<TRANS, TA>(s, m, r, k, alpha, A, lda, B, ldb, beta, C, ldc, &status) == 0)
 		return status;
 	if (gemm_thin_mfma<TRANS, TA>(s, m, r, k, alpha, A, lda, B, ldb, beta, C, ldc, work, work_bytes, &status) == 0)
