@@ -164,14 +164,21 @@ __device__ __forceinline__ int await(const PfArgs &p, const sa_gu *f1, const sa_
 // Every thread's stores become visible at agent scope, then the counter is
 // raised.  Each wave waits for its own stores to complete before the
 // barrier; thread 0's agent-scope release then covers them all, so the L2
-// write-back runs once per item rather than once per wave.
+// write-back runs once per item rather than once per wave.  The wait for that
+// write-back is written out: the compiler takes the wait before the barrier
+// for proof that nothing is outstanding and drops the one of a release
+// fence or store that follows it, and the counter then reaches another XCD
+// before the data has left this one's L2.
 __device__ __forceinline__ void publish(sa_gu *f, unsigned v)
 {
 	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
 	__builtin_amdgcn_s_waitcnt(0);
 	__syncthreads();
-	if (threadIdx.x == 0)
-		__hip_atomic_store(f, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+	if (threadIdx.x == 0) {
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+		__builtin_amdgcn_s_waitcnt(0);
+		__hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
 }
 
 // acc += Pr Pc^T over the columns 64 t0 .. 64 t1 - 1 of two block rows, for

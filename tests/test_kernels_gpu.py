@@ -361,6 +361,66 @@ def test_dpotrf_tile_block_edges(K, n, wg):
     assert info.get() == 0 and np.array_equal(dA2.download(), got)
 
 
+@pytest.mark.parametrize("n,pad", [(130, 0), (512, 0), (768, 0), (960, 1), (1024, 0)])
+def test_dpotrf_tile_beside_writing_kernels(K, n, pad):
+    # four factorisations with their inverses on streams of their own, beside
+    # tile products that keep dirtying the caches: the same bits as alone.
+    # The workspace, W, Linv and the strict upper triangle hold NaN before every call, so
+    # that whatever is read before its workgroup has published it shows.
+    print(f"dpotrf_tile beside products n={n} pad={pad}", flush=True)
+    import ctypes as C
+    L = K.lib()
+    rng = np.random.default_rng(n + pad)
+    nan, ld, wb = float("nan"), n + pad, L.sa_dpotrf_tile_worksize(n)
+    streams = []
+    for _ in range(6):
+        s = C.c_void_p()
+        K.check(L.sa_stream_create(C.byref(s)), "stream")
+        streams.append(s)
+    sets = []
+    for i in range(4):
+        A = spd(rng, n)
+        A[np.triu_indices(n, 1)] = np.nan
+        d = {"A0": dev(K, A, ld), "A": K.DeviceArray(n, n, ld=ld), "X": K.DeviceArray(n, n, ld=ld),
+             "W": K.DeviceArray(n, n, ld=ld), "ws": K.DeviceArray(wb // 8, 1), "info": K.DeviceInt(-7)}
+        sets.append(d)
+    g = 1024
+    P, Q = dev(K, rng.uniform(-1, 1, (g, g))), dev(K, rng.uniform(-1, 1, (g, g)))
+    outs = [K.DeviceArray(g, g) for _ in range(2)]
+
+    def factor(d, s):
+        K.check(L.sa_dlaset(s, wb // 8, 1, nan, nan, d["ws"].ptr, wb // 8), "fill")
+        for x in ("W", "X"):
+            K.check(L.sa_dlaset(s, n, n, nan, nan, d[x].ptr, ld), "fill")
+        K.check(L.sa_dlacpy(s, n, n, d["A0"].ptr, ld, d["A"].ptr, ld), "copy")
+        K.check(L.sa_dpotrf_tile_wg(s, n, d["A"].ptr, ld, d["X"].ptr, ld, d["W"].ptr, ld, d["info"].ptr, d["ws"].ptr,
+                                    wb, 63), "dpotrf_tile")
+
+    def result(d):
+        assert d["info"].get() == 0
+        d["info"].set(-7)
+        return np.tril(d["A"].download()), d["X"].download(), d["W"].download()
+
+    ref = []
+    for d in sets:
+        factor(d, streams[0])
+        K.sync()
+        ref.append(result(d))
+        assert np.isfinite(ref[-1][0]).all() and np.array_equal(ref[-1][1], ref[-1][2].T)
+    for rep in range(20):
+        for _ in range(4):
+            for s, c in zip(streams[4:], outs):
+                K.dgemm_nt(g, g, g, 1.0, P.ptr, g, Q.ptr, g, 0.0, c.ptr, g, stream=s)
+        for d, s in zip(sets, streams):
+            factor(d, s)
+        K.sync()
+        for d, r in zip(sets, ref):
+            for a, b in zip(result(d), r):
+                assert np.array_equal(a, b), rep
+    for s in streams:
+        K.check(L.sa_stream_destroy(s), "destroy")
+
+
 def test_tile_limit_and_large_tile_inverse(K):
     # tiles past the single-launch limit: sa_dpotrf_tile refuses them, and
     # sa_dtrtri_tile inverts them by substitution

@@ -3,9 +3,10 @@ solve requests of mixed sizes with re-solves, HBM-budget admission and
 eviction, and the same result for a request alone and in the mix.
 
 Each request must reach normwise backward error <= 1e-14 (the FP64 bar)
-and agree with an FP64 solve to cond(A) * 1e-14; alone versus in the mix
-the solutions must agree to 1e-13 relative (the arithmetic of a request
-does not depend on what else runs, so they are expected to be equal)."""
+and agree with an FP64 solve to cond(A) * 1e-14; alone and in the mix it
+must give the same bits after the same number of refinement steps (the
+arithmetic of a request does not depend on what else runs; refinement would
+repair a factor that is wrong in a few elements, its step count shows it)."""
 import os
 import tempfile
 
@@ -69,6 +70,7 @@ def test_same_result_alone_and_in_the_mix(env):
     reqs = inp.requests(tr, alone=True)
     R.serve(S.config(budget_gb=20, slots=1, nb=512), reqs)
     alone = [x.download() for x in inp.X]
+    steps = [q.iterations for q in reqs]
     # in the mix: all arrive together, four in service
     for x in inp.X:
         K.check(K.lib().sa_dlaset(None, x.m, x.n, 0.0, 0.0, x.ptr, x.ld))
@@ -76,9 +78,9 @@ def test_same_result_alone_and_in_the_mix(env):
     st = R.serve(S.config(budget_gb=20, slots=4, nb=512), reqs)
     assert st.max_inflight >= 2
     check_solutions(K, inp, tr, reqs)
+    assert [q.iterations for q in reqs] == steps
     for i, x in enumerate(inp.X):
-        mixed = x.download()
-        assert np.linalg.norm(mixed - alone[i]) / np.linalg.norm(alone[i]) <= 1e-13, i
+        assert np.array_equal(x.download(), alone[i]), i
     inp.free()
 
 
