@@ -124,6 +124,12 @@ int sa_dpotrf_tile_wg(hipStream_t stream, int n, double *A, int lda, double *Lin
                       int *dev_info, void *work, size_t work_bytes, int workgroups);
 size_t sa_dpotrf_tile_worksize(int n);
 int sa_dpotrf_tile_maxn(void);
+/* sa_dpotrf_tile_wg whose inverse items wait no longer than the factorisation
+ * takes: a wait still open then gives up, as any wait does after seconds,
+ * and *dev_info is -1 (W and Linv are then not the inverse).  For tests of
+ * that report. */
+int sa_dpotrf_tile_cut(hipStream_t stream, int n, double *A, int lda, double *Linv, int ldl, double *W, int ldw,
+                       int *dev_info, void *work, size_t work_bytes, int workgroups);
 
 /* Allocation-free variant of sa_dpotrf_tile: the same kernels, with the
  * workspace in a device array the library holds on each GPU for the

@@ -66,7 +66,10 @@
 // an abort flag, after which no wait waits any more: every workgroup runs
 // through its items on whatever memory holds (in bounds all the same), the
 // grid drains and the factorisation reports info = -1, so a fault of the
-// ordering shows as an error, not as a hung device.
+// ordering shows as an error, not as a hung device.  The chain writes info
+// while the last inverse items may still run; a wait of theirs that gives up
+// after that writes -1 itself (give_up).  Inverting a factored tile has no
+// info to report in.
 //
 // Visibility across workgroups (possibly on different XCDs, each with its own
 // L2) uses agent-scope release fences before a counter is raised and an
@@ -115,6 +118,7 @@ struct PfArgs {
 	long ldi;
 	sa_gd *Dinv;      // nb blocks of 64x64 (ld 64)
 	sa_gu *flags;
+	unsigned stop;      // bits of the abort word that end a wait: ABORT_GAVE_UP
 	int *info;
 	__device__ sa_gu *rowl(int i) const { return flags + FLAG_STRIDE * i; }          // L(i,t) final for t < value
 	__device__ sa_gu *diag(int i) const { return flags + FLAG_STRIDE * (nb + i); }   // A(i,i) but for t = i - 1
@@ -138,6 +142,22 @@ __device__ __forceinline__ unsigned flag_read(const sa_gu *f)
 // item takes tens of microseconds).
 constexpr unsigned SPIN_LIMIT = 1u << 22;
 
+// The abort word: a wait gave up; the chain has written info (and what it
+// wrote is in memory).  Each side sets its bit and looks at the other's in one
+// atomic step, so one of them sees both and the -1 is the last store to info.
+constexpr unsigned ABORT_GAVE_UP = 1, ABORT_REPORTED = 2;
+
+__device__ __forceinline__ unsigned abort_or(const PfArgs &p, unsigned bit)
+{
+	return __hip_atomic_fetch_or(p.abortf(), bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void give_up(const PfArgs &p)
+{
+	if ((threadIdx.x & 63) == 0 && (abort_or(p, ABORT_GAVE_UP) & ABORT_REPORTED) && p.info)
+		*p.info = -1;
+}
+
 // One wave waits until both counters have reached v (or the run is
 // abandoned) and then sees the data published before they were raised.
 // Returns the smaller counter, at least v.
@@ -150,8 +170,8 @@ __device__ __forceinline__ int await(const PfArgs &p, const sa_gu *f1, const sa_
 		m = __builtin_amdgcn_readfirstlane(a < b ? a : b);
 		if (m >= v)
 			break;
-		if (__builtin_amdgcn_readfirstlane((int)flag_read(p.abortf())) || ++it > SPIN_LIMIT) {
-			__hip_atomic_store(p.abortf(), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		if (((unsigned)__builtin_amdgcn_readfirstlane((int)flag_read(p.abortf())) & p.stop) || ++it > SPIN_LIMIT) {
+			give_up(p);
 			m = v;
 			break;
 		}
@@ -483,6 +503,8 @@ __device__ __forceinline__ void run_chain(const PfArgs &p, double *S, double *Li
 		store_inv64<double>(Li, (double *)(p.Dinv + 4096L * j));
 		store_lower64<double>(wj, S, (double *)(p.A + 64 * j + 64L * j * p.lda), p.lda);
 		if (j + 1 == p.nb) {
+			if (threadIdx.x == 0)
+				*p.info = first_bad;     // in memory once D(j) is published
 			publish(p.dfin(j), 1u);
 			break;
 		}
@@ -563,8 +585,12 @@ __device__ __forceinline__ void run_chain(const PfArgs &p, double *S, double *Li
 		}
 		__syncthreads();
 	}
-	if (threadIdx.x == 0)
-		*p.info = flag_read(p.abortf()) ? -1 : first_bad;
+	if (threadIdx.x == 0) {
+		if (p.nb == 0)
+			*p.info = 0;
+		else if (abort_or(p, ABORT_REPORTED) & ABORT_GAVE_UP)
+			*p.info = -1;
+	}
 }
 
 // ---- the bulk order --------------------------------------------------------
@@ -731,7 +757,7 @@ long count_items(const PfOrder &o)
 // holds the factor.  W (and Linv, optional) receive the inverse when W is
 // given.  bulk: workgroups for the bulk items (<= 0: max_bulk()).
 int launch_tile(hipStream_t s, int n, double *A, int lda, int *dev_info, void *work, double *W, int ldw,
-                double *Linv, int ldi, int factor, int bulk = 0)
+                double *Linv, int ldi, int factor, int bulk = 0, unsigned stop = ABORT_GAVE_UP)
 {
 	const int nb = n > 0 ? (n + 63) / 64 : 0;
 	char *ws = (char *)work;
@@ -749,6 +775,7 @@ int launch_tile(hipStream_t s, int n, double *A, int lda, int *dev_info, void *w
 	p.ldi = ldi;
 	p.Dinv = (sa_gd *)ws;
 	p.flags = (sa_gu *)(ws + align256((size_t)(nb ? nb : 1) * 4096 * sizeof(double)));
+	p.stop = stop;
 	p.info = dev_info;
 	if (nb == 0) {
 		if (!factor)
@@ -789,14 +816,27 @@ extern "C" size_t sa_dpotrf_tile_worksize(int n)
 
 extern "C" int sa_dpotrf_tile_maxn(void) { return PF_MAXN; }
 
-extern "C" int sa_dpotrf_tile_wg(hipStream_t s, int n, double *A, int lda, double *Linv, int ldl, double *W,
-                                 int ldw, int *dev_info, void *work, size_t work_bytes, int workgroups)
+static int potrf_tile(hipStream_t s, int n, double *A, int lda, double *Linv, int ldl, double *W, int ldw,
+                      int *dev_info, void *work, size_t work_bytes, int workgroups, unsigned stop)
 {
 	if (n < 0 || n > PF_MAXN || lda < (n > 1 ? n : 1) || !dev_info || !work ||
 	    work_bytes < sa_dpotrf_tile_worksize(n) || (Linv && !W) ||
 	    (W && ldw < (n > 1 ? n : 1)) || (Linv && ldl < (n > 1 ? n : 1)))
 		return -EINVAL;
-	return launch_tile(s, n, A, lda, dev_info, work, W, ldw, Linv, ldl, 1, workgroups);
+	return launch_tile(s, n, A, lda, dev_info, work, W, ldw, Linv, ldl, 1, workgroups, stop);
+}
+
+extern "C" int sa_dpotrf_tile_wg(hipStream_t s, int n, double *A, int lda, double *Linv, int ldl, double *W,
+                                 int ldw, int *dev_info, void *work, size_t work_bytes, int workgroups)
+{
+	return potrf_tile(s, n, A, lda, Linv, ldl, W, ldw, dev_info, work, work_bytes, workgroups, ABORT_GAVE_UP);
+}
+
+extern "C" int sa_dpotrf_tile_cut(hipStream_t s, int n, double *A, int lda, double *Linv, int ldl, double *W,
+                                  int ldw, int *dev_info, void *work, size_t work_bytes, int workgroups)
+{
+	return potrf_tile(s, n, A, lda, Linv, ldl, W, ldw, dev_info, work, work_bytes, workgroups,
+	                  ABORT_GAVE_UP | ABORT_REPORTED);
 }
 
 extern "C" int sa_dpotrf_tile(hipStream_t s, int n, double *A, int lda, double *Linv, int ldl, double *W, int ldw,

@@ -421,6 +421,32 @@ def test_dpotrf_tile_beside_writing_kernels(K, n, pad):
         K.check(L.sa_stream_destroy(s), "destroy")
 
 
+def test_dpotrf_tile_reports_inverse_that_gave_up(K):
+    # waits of the inverse items that are given up after the chain has
+    # reported: info is -1, or the inverse is whole; the factor always is
+    n = 1024
+    L = K.lib()
+    rng = np.random.default_rng(77)
+    A = spd(rng, n)
+    wb = L.sa_dpotrf_tile_worksize(n)
+    ws, info = K.DeviceArray(wb // 8, 1), K.DeviceInt(-7)
+    dW = K.DeviceArray(n, n)
+    seen = []
+    # with 127 or 255 bulk workgroups some wait is open then in 4 runs of 5
+    for f, wg in [(L.sa_dpotrf_tile_wg, 31)] + [(L.sa_dpotrf_tile_cut, w) for w in (31, 127, 255) * 8]:
+        print(f"dpotrf_tile_cut workgroups={wg}", flush=True)
+        dA = dev(K, A)
+        K.check(L.sa_dlaset(None, n, n, float("nan"), float("nan"), dW.ptr, n), "fill")
+        K.check(f(None, n, dA.ptr, n, None, 0, dW.ptr, n, info.ptr, ws.ptr, wb, wg), "dpotrf_tile")
+        K.sync()
+        got, W, v = dA.download(), dW.download(), info.get()
+        if not seen:
+            ref, Wref = got, W
+        seen.append(v)
+        assert np.array_equal(got, ref) and (v == -1 or (v == 0 and np.array_equal(W, Wref))), seen
+    assert seen[0] == 0 and -1 in seen, seen
+
+
 def test_tile_limit_and_large_tile_inverse(K):
     # tiles past the single-launch limit: sa_dpotrf_tile refuses them, and
     # sa_dtrtri_tile inverts them by substitution
