@@ -158,39 +158,35 @@ __device__ __forceinline__ typename V4<T>::type ld16(const T *P)
 	return acc;
 }
 
-// 1/sqrt(d) to full precision: the hardware estimate r (about 24 bits in
-// either type) and e = 1 - d r^2; for double one third-order step
-// r + r e (1/2 + 3/8 e), whose error is of order e^3, for float one Newton
-// step.
-__device__ __forceinline__ double rsqrt_nr(double d)
-{
-	const double r = __builtin_amdgcn_rsq(d);
-	const double e = fma(-d * r, r, 1.0);
-	return fma(r * e, fma(0.375, e, 0.5), r);
-}
+// The hardware estimate r of 1/sqrt(d) (about 24 bits in either type) and
+// e = 1 - d r^2, from which both of a column's scalings come to full
+// precision: 1/sqrt(d), for double by a third-order step
+// r + r e (1/2 + 3/8 e), whose error is of order e^3, for float by a Newton
+// step; and x / d = x r^2 / (1 - e), for double x r^2 (1 + e + e^2), for
+// float x r^2 (1 + e).  x r is formed first: |x| <= sqrt(d a) for a the
+// diagonal entry of x's row, so it stays in range, and x r^2 as long as
+// sqrt(a / d) does, which only a subnormal d can break.  1/d does not: it
+// overflows for an FP64 pivot below 2^-1024, and from 2^126 on an FP32 one's
+// is a subnormal that the reciprocal instruction flushes, which would leave
+// the elimination out.
+__device__ __forceinline__ double rsqrt_est(double d) { return __builtin_amdgcn_rsq(d); }
+__device__ __forceinline__ float rsqrt_est(float d) { return __builtin_amdgcn_rsqf(d); }
 
-__device__ __forceinline__ float rsqrt_nr(float d)
-{
-	const float r = __builtin_amdgcn_rsqf(d);
-	const float h = 0.5f * d;
-	return fmaf(r, fmaf(-h * r, r, 0.5f), r);
-}
+__device__ __forceinline__ double rsqrt_err(double d, double r) { return fma(-d * r, r, 1.0); }
+__device__ __forceinline__ float rsqrt_err(float d, float r) { return fmaf(-d * r, r, 1.0f); }
 
-// The hardware estimate of 1/d, and x / d from such an estimate y and
-// e = 1 - d y: x y (1 + e + e^2) for double (error of order e^3), x y (1 + e)
-// for float.
-__device__ __forceinline__ double rcp_est(double d) { return __builtin_amdgcn_rcp(d); }
-__device__ __forceinline__ float rcp_est(float d) { return __builtin_amdgcn_rcpf(d); }
+__device__ __forceinline__ double rsqrt_nr(double r, double e) { return fma(r * e, fma(0.375, e, 0.5), r); }
+__device__ __forceinline__ float rsqrt_nr(float r, float e) { return fmaf(r, 0.5f * e, r); }
 
-__device__ __forceinline__ double quot_nr(double x, double d, double y)
+__device__ __forceinline__ double quot_nr(double x, double r, double e)
 {
-	const double e = fma(-d, y, 1.0), x0 = x * y;
+	const double x0 = x * r * r;
 	return fma(x0, fma(e, e, e), x0);
 }
 
-__device__ __forceinline__ float quot_nr(float x, float d, float y)
+__device__ __forceinline__ float quot_nr(float x, float r, float e)
 {
-	const float e = fmaf(-d, y, 1.0f), x0 = x * y;
+	const float x0 = x * r * r;
 	return fmaf(x0, e, x0);
 }
 
@@ -212,7 +208,7 @@ __device__ __forceinline__ int potrf16_regs(T (&x)[16], F done)
 #pragma unroll
 	for (int k = 0; k < 16; k++) {
 		const T d = bcast_rl(x[k], k);
-		const T y = rcp_est(d);
+		const T r = rsqrt_est(d);
 		__builtin_amdgcn_sched_barrier(0);
 		// all multipliers of the column in scalar registers, behind the
 		// estimate's latency and before the first is used: a readlane's
@@ -221,13 +217,13 @@ __device__ __forceinline__ int potrf16_regs(T (&x)[16], F done)
 #pragma unroll
 		for (int j = k + 1; j < 16; j++)
 			m[j] = bcast_rl(x[k], j);
-		const T z = quot_nr(x[k], d, y);
+		const T e = rsqrt_err(d, r), z = quot_nr(x[k], r, e);
 		bad |= __ballot(!(x[k] > T(0))) & (1ull << k);
 		__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
 		for (int j = k + 1; j < 16; j++)
 			x[j] -= z * m[j];
-		x[k] *= rsqrt_nr(d);
+		x[k] *= rsqrt_nr(r, e);
 		done(k, x[k]);
 	}
 	return __ffsll((long long)bad);

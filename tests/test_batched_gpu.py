@@ -226,6 +226,57 @@ def test_ir_fp32_breakdown_falls_back_to_fp64(B):
     batch.free()
 
 
+def scaled_systems(batch, e):
+    """Fills the batch with 2^e L L^T and right-hand sides 2^e b for sparse
+    L with small integers (diagonal 2..23, so the first pivot of each column
+    group is exact) and b = L L^T 1; returns the Ls."""
+    from starpu_amd import kernels as K
+    rng = np.random.default_rng(3)
+    Ls = []
+    for i, v in enumerate(int(n) for n in batch.n):
+        L = np.tril(rng.integers(-1, 2, (v, v)) * (rng.random((v, v)) < 3.0 / v), -1).astype(float)
+        L += np.diag(rng.choice([2.0, 4.0, 16.0, 23.0], v))
+        A = np.asfortranarray(np.ldexp(L @ L.T, e))
+        b = np.ldexp(L @ L.T @ np.ones(v), e)
+        assert np.isfinite(A).all() and (np.ldexp(A, -e) == L @ L.T).all()
+        K.check(K.lib().sa_memcpy_h2d(batch.A0.ptr + int(batch.offA[i]) * 8, A.ctypes.data, A.nbytes))
+        K.check(K.lib().sa_memcpy_h2d(batch.B0.ptr + int(batch.offB[i]) * 8, b.ctypes.data, b.nbytes))
+        Ls.append(L)
+    batch.restore()
+    return Ls
+
+
+@pytest.mark.parametrize("e", [-1046, -1030, -1022, 0, 1000, 1014])
+def test_pivots_at_the_ends_of_the_fp64_range(B, e):
+    # pivots 2^e (4..529): subnormal, and where their reciprocal is; L is
+    # 2^(e/2) times small integers, so nothing else leaves the range.  Bar:
+    # n eps times a condition of a few hundred, as 1e-12 elsewhere
+    batch = B.Batch([5, 16, 40, 64, 100, 130], nrhs=1, seed=6)
+    Ls = scaled_systems(batch, e)
+    batch.launch(8)
+    assert (batch.infos() == 0).all(), batch.infos()
+    for i, L in enumerate(Ls):
+        got = np.ldexp(batch.system(i)[3], -e // 2)
+        assert np.linalg.norm(got - L) <= 1e-12 * np.linalg.norm(L), (i, np.linalg.norm(got - L))
+    batch.free()
+
+
+@pytest.mark.parametrize("e", [-124, 0, 110, 118])
+def test_pivots_at_the_ends_of_the_fp32_range(B, e):
+    # the FP32 factor's pivots 2^e (4..529), up to 2^127: where the
+    # reciprocal of one is subnormal the elimination must not be left out,
+    # which costs refinement steps or the solution
+    batch = B.Batch([5, 16, 40, 64, 100, 130], nrhs=1, seed=6, ir=True)
+    scaled_systems(batch, e)
+    batch.launch_ir(8)
+    assert (batch.infos() == 0).all(), batch.infos()
+    for i in range(len(batch.n)):
+        x, it, be = batch.ir_result(i)
+        assert it[0] <= 4 and be[0] <= 1e-14, (i, it, be)
+        assert np.linalg.norm(x[:, 0] - 1.0) <= 1e-10 * np.sqrt(len(x)), i
+    batch.free()
+
+
 def test_ir_graph_replays_match_eager(B):
     import ctypes as C
     from starpu_amd import kernels as K
