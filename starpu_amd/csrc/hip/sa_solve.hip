@@ -750,12 +750,16 @@ int gemm_thin_mfma(hipStream_t s, int m, int r, int k, double alpha, const TA *A
 // 27.1 / 29.0 and 31.9 / 33.6 at 4096 rows, 49.4 / 51.3 and 42.1 / 49.4 at
 // 8192; 64 at 4096 rows 39.8 / 43.9 and 33.5 / 39.8.  Below the rows the MFMA
 // form takes, it wins whatever their number (1024 rows: 64 17.1 / 15.6 and
-// 32.4 / 34.5, 512 58 / 74 and 155 / 180).
+// 32.4 / 34.5, 512 58 / 74 and 155 / 180).  A workgroup takes the whole of k,
+// so past k = 2048 the split wins on short products: back to back, 16
+// right-hand sides, 512 / 1024 / 4096 rows (NN), k = 2048 19.0 / 19.4 / 23.2
+// against 19.6 / 24.1 / 28.4, k = 3072 28.0 / 28.6 / 33.1 against 27.9 / 26.5 /
+// 33.4, k = 4096 35.0 / 35.8 / 42.3 against 31.6 / 28.0 / 46.3.
 constexpr int THIN_ROWS_MAX_K = 2048, THIN_ROWS_MAX_M = 12288;
 
 bool thin_rows_wins(int m, int r, int k)
 {
-	return k <= THIN_ROWS_MAX_K && (m < MFMA_MIN_M || (long)m * ((r + 15) / 16) <= THIN_ROWS_MAX_M);
+	return k <= THIN_ROWS_MAX_K && (m < thin_mfma_min_m() || (long)m * ((r + 15) / 16) <= THIN_ROWS_MAX_M);
 }
 
 template <bool TRANS, typename TA = double>

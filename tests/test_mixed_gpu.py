@@ -9,6 +9,8 @@ relative to |A|^T |B|; integer inputs small enough to be exact in bf16 and
 in FP32 sums are bit-exact; the refined solution reaches normwise backward
 error <= 1e-14, the FP64 bar."""
 import os
+import subprocess
+import sys
 import tempfile
 
 import numpy as np
@@ -295,6 +297,37 @@ def test_thin_rows_k_shares(K, dtype, m, r, k):
         dC = K.DeviceArray.from_host(C0)
         K.check(f(None, m, r, k, -1.0, dA.ptr, dA.ld, dB.ptr, dB.ld, 2.0, dC.ptr, dC.ld, None, 0), "thin")
         assert np.array_equal(dC.download(), exp)
+
+
+@pytest.mark.parametrize("min_m,m,r,split", [("512", 1024, 256, True), ("512", 1024, 16, False), ("", 1024, 256, False),
+                                             ("65536", 16384, 16, False), ("", 16384, 16, True)])
+def test_thin_mfma_min_m_moves_the_limit_of_the_one_launch_form(K, min_m, m, r, split):
+    # SA_THIN_MFMA_MIN_M, read once per process: from that many rows on a wide
+    # enough product takes the split form, which leaves its partial sums in
+    # the workspace; the one-launch form does not touch it
+    code = f"""
+import numpy as np
+from starpu_amd import kernels as K
+L, m, r, k = K.lib(), {m}, {r}, 512
+rng = np.random.default_rng(1)
+A, B = rng.integers(-9, 10, (m, k)).astype(float), rng.integers(-9, 10, (k, r)).astype(float)
+dA, dB, dC = K.DeviceArray.from_host(A), K.DeviceArray.from_host(B), K.DeviceArray(m, r)
+wb = max(8, L.sa_dgemm_thin_worksize(m, r, k))
+ws = K.DeviceArray(wb // 8, 1)
+K.check(L.sa_dlaset(None, wb // 8, 1, float("nan"), float("nan"), ws.ptr, wb // 8))
+K.check(L.sa_dgemm_nn(None, m, r, k, 1.0, dA.ptr, m, dB.ptr, k, 0.0, dC.ptr, m, ws.ptr, wb))
+K.sync()
+assert np.array_equal(dC.download(), A @ B)
+print("split", not np.isnan(ws.download()).all())
+"""
+    env = dict(os.environ)
+    env.pop("SA_THIN_MFMA_MIN_M", None)
+    if min_m:
+        env["SA_THIN_MFMA_MIN_M"] = min_m
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.split() == ["split", str(split)]
 
 
 @pytest.mark.parametrize("n,r", [(1, 1), (17, 3), (255, 16), (256, 16), (300, 17), (1000, 5), (2049, 16),
