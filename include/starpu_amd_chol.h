@@ -181,7 +181,8 @@ struct chol_serve_request {
 	double start_us, finish_us;  /* service start and completion, from the start of the trace */
 	double berr;                 /* final normwise backward error */
 	int iterations;              /* solves with the FP32 factor */
-	int status;                  /* 0, a pivot column (not SPD) or a negative errno */
+	int status;                  /* 0, a pivot column (not SPD) or a negative errno; -ERANGE: the
+	                              * refinement ended above cfg->tol (X holds its last iterate) */
 	int factored;                /* 1 if this request ran the factorisation */
 	double factor_start_us, factor_end_us;  /* its factorisation (when factored), from the start of the trace */
 };

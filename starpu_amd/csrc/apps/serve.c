@@ -261,6 +261,9 @@ static void *worker(void *arg)
 				q->status = chol_mixed_refine(&e->f, q->A, q->lda, q->B, q->ldb, q->nrhs, q->X, q->ldx, cfg->tol,
 				                              cfg->maxiter, s, work, wb, &q->iterations, &q->berr, NULL, 0);
 				sa_stream_sync(s);
+				/* refinement that ended above the target is no solution */
+				if (q->status == 0 && !(q->berr <= cfg->tol))
+					q->status = -ERANGE;
 			}
 		}
 		q->finish_us = now_us() - S->t0;

@@ -120,3 +120,19 @@ def test_request_larger_than_budget_is_rejected(env):
     assert reqs[1].status == 0 and reqs[1].berr <= 1e-14
     assert st.factorizations == 1
     inp.free()
+
+
+def test_request_that_misses_its_target_is_reported(env):
+    # a target below rounding: the refinement ends at its step limit, with a
+    # solution that is as good as FP64 allows
+    K, R, S = env
+    tr = S.Trace(n=[512, 256], nrhs=[2, 1], matrix=[0, 1], arrival_us=[0.0, 0.0], matrix_n=[512, 256])
+    inp = S.Inputs(tr, shift=0.01, seed=41)
+    reqs = inp.requests(tr)
+    R.serve(S.config(budget_gb=20, slots=2, nb=256, tol=1e-30, maxiter=3), reqs)
+    for i, q in enumerate(reqs):
+        assert q.status == -34 and 0 < q.berr <= 1e-14 and q.iterations == 4, (q.status, q.berr, q.iterations)   # -ERANGE
+        A, b, x = inp.A[i].download(), inp.B[i].download(), inp.X[i].download()
+        ref = np.linalg.solve(A, b)
+        assert np.linalg.norm(x - ref) / np.linalg.norm(ref) < 10 * np.linalg.cond(A) * 1e-14
+    inp.free()
