@@ -112,8 +112,21 @@ static int evict_one(struct server *S)
 	return 1;
 }
 
+/* Evict until the budget and the node's memory, which the runtime's
+ * replicates share, hold `need` more bytes, and reserve them there. */
+static int make_room(struct server *S, size_t need)
+{
+	while (S->used + (double)need > S->cfg->budget_bytes)
+		if (!evict_one(S))
+			return 0;
+	while (starpu_memory_allocate((unsigned)S->hip_node, need, 0) != 0)
+		if (!evict_one(S))
+			return 0;
+	return 1;
+}
+
 /* Admit request r (mutex held): reserve its bytes, pin or create its cache
- * entry.  Returns 0 if the budget cannot hold it now. */
+ * entry.  Returns 0 if the budget cannot hold it now, -1 if it never can. */
 static int try_admit(struct server *S, int r, struct cache_entry **entry, size_t *work_bytes, int *creator)
 {
 	struct chol_serve_request *q = &S->req[r];
@@ -123,17 +136,19 @@ static int try_admit(struct server *S, int r, struct cache_entry **entry, size_t
 		e = NULL;
 	const size_t wb = chol_mixed_refine_worksize(q->n, nbk, q->nrhs);
 	const size_t fb = e ? 0 : chol_mixed_factor_bytes(q->n, nbk);
-	const double need = (double)wb + (double)fb;
+	const double need = (double)wb + (double)fb, whole = need + (e ? (double)e->bytes : 0.0);
 	const long long node_total = starpu_memory_get_total((unsigned)S->hip_node);
-	if (need > S->cfg->budget_bytes || (node_total >= 0 && need > (double)node_total))
+	if (whole > S->cfg->budget_bytes || (node_total >= 0 && whole > (double)node_total))
 		return -1;          /* can never fit */
-	while (S->used + need > S->cfg->budget_bytes)
-		if (!evict_one(S))
-			return 0;
-	/* the node's budget, shared with the runtime's replicates */
-	while (starpu_memory_allocate((unsigned)S->hip_node, (size_t)need, 0) != 0)
-		if (!evict_one(S))
-			return 0;
+	/* pinned before room is made: the factor this request reuses may be
+	 * the least recently used one */
+	if (e)
+		e->pins++;
+	if (!make_room(S, wb + fb)) {
+		if (e)
+			e->pins--;
+		return 0;
+	}
 	if (!e) {
 		/* a failed entry for this matrix is replaced */
 		struct cache_entry *old = cache_find(S, q->matrix);
@@ -147,12 +162,12 @@ static int try_admit(struct server *S, int r, struct cache_entry **entry, size_t
 		if (!e)
 			return 0;
 		e->bytes = fb;
+		e->pins = 1;
 		*creator = 1;
 	} else {
 		*creator = 0;
 		S->st.cache_hits++;
 	}
-	e->pins++;
 	S->used += need;
 	if (S->used > S->peak)
 		S->peak = S->used;

@@ -136,3 +136,34 @@ def test_request_that_misses_its_target_is_reported(env):
         ref = np.linalg.solve(A, b)
         assert np.linalg.norm(x - ref) / np.linalg.norm(ref) < 10 * np.linalg.cond(A) * 1e-14
     inp.free()
+
+
+def test_resolve_does_not_evict_the_factor_it_reuses(env):
+    # the least recently used factor is the one that the third request
+    # reuses, and its larger work area needs room: the other factor goes.  The
+    # fourth request's work area does not fit beside its factor at all
+    K, R, S = env
+    import ctypes
+    lib = R.chol()
+    lib.chol_mixed_factor_bytes.restype = lib.chol_mixed_refine_worksize.restype = ctypes.c_size_t
+    n, r = 1024, 32
+    fb = lib.chol_mixed_factor_bytes(n, 4)
+
+    def wb(nrhs):
+        return lib.chol_mixed_refine_worksize(n, 4, nrhs)
+
+    budget = 2 * fb + wb(r) - 1
+    big = r
+    while wb(big) + fb <= budget:
+        big += 1
+    assert wb(big) <= budget                # fits alone, as the check of a resident factor's request once was
+    tr = S.Trace(n=[n] * 5, nrhs=[1, 1, r, big, r], matrix=[0, 1, 0, 0, 0], arrival_us=[0.0] * 5, matrix_n=[n] * 2)
+    inp = S.Inputs(tr, shift=0.01, seed=51)
+    reqs = inp.requests(tr)
+    st = R.serve(S.config(budget_gb=budget / 1e9, slots=1, nb=256), reqs)
+    print([q.status for q in reqs], st.evictions, st.cache_hits, st.factorizations, flush=True)
+    assert reqs[3].status == -12                                       # -ENOMEM
+    check_solutions(K, inp, tr, reqs, idx=[0, 1, 2, 4])
+    assert [q.factored for q in reqs] == [1, 1, 0, 0, 0]
+    assert (st.evictions, st.cache_hits, st.factorizations) == (1, 2, 2) and st.peak_bytes <= budget
+    inp.free()
