@@ -355,8 +355,8 @@ __device__ __forceinline__ int block_core64(T *__restrict__ S, T *__restrict__ L
 		// wave q = 1..3 keeps the sum of the next block of its inverse column
 		V t = zero4<T>();
 		const int Jc = wave - 1;
-		// not unrolled: one copy of the panel code, 16 columns of it, stays in
-		// the instruction cache
+		// unrolled: the conditions on J below fold, at the price of four
+		// copies of the panel code
 #pragma unroll
 		for (int J = 0; J < 4; J++) {
 			if (wave == 0) {

@@ -64,10 +64,11 @@ struct Frag<MODE_BF16X3> {
 // conversion and LDS stores of chunk c + 2 and the loads of chunk c + 4: a
 // wave issues in order and there is one per SIMD, so what does not stand
 // between MFMAs stands beside them.  One barrier a chunk.  Products of 1024^3
-// alone (us): FP32 23.1, BF16x3 18.3, BF16 11.0; of 469^3: 13.1, 10.9, 7.8.
-// With loads, conversion and stores in groups around the MFMAs, 128x128
-// workgroups and a 16-byte alignment they took 76.4, 37.7 and 22.0; without
-// the alignment, operands straight from L2, 469^3 took 56.
+// alone (us) with 64x64 / 128x128 tiles: FP32 20.9 / 67.6, BF16x3 14.9 / 32.1,
+// BF16 9.6 / 19.3; of 469^3 with 64x64: 12.8, 10.1, 7.5.  With loads, conversion
+// and stores in groups around the MFMAs, 128x128 workgroups and a 16-byte
+// alignment 1024^3 took 76.4, 37.7 and 22.0; without the alignment, operands
+// straight from L2, 469^3 took 56.
 template <int MODE> struct StageT { typedef __bf16 type; static constexpr int planes = MODE == MODE_BF16X3 ? 2 : 1, col = 40; };
 template <> struct StageT<MODE_F32> { typedef float type; static constexpr int planes = 1, col = 36; };
 
@@ -644,11 +645,12 @@ void k_split_bf16x2(int m, int n, const float *__restrict__ A, long lda, __bf16 
 
 // 64x64 workgroup tiles up to products that give 192 workgroups of 128x128
 // (FP32) or 64 (BF16 forms): four times the workgroups, three on a compute
-// unit against one.  Alone, 1024^3 FP32 takes 23.1 us against 67.9 and with
-// four launches in flight 20.8 against 35.0; BF16x3, where the 64x64 form
-// spends its time on LDS reads, 18.3 against 31.7 alone, but the N=32768
-// factorisation on 1024 tiles with four hardware queues runs its 128x128
-// form in 90.7 ms (solve included) against 95.5, 512 tiles the 64x64 form.
+// unit against one.  Alone, 1024^3 FP32 takes 20.9 us against 67.6 and with
+// four launches in flight on operands of their own 20.8 against 35.0; BF16x3,
+// where the 64x64 form spends its time on LDS reads, 14.9 against 32.1 alone,
+// but the N=32768 factorisation on 1024 tiles with four hardware queues runs
+// its 128x128 form in 90.7 ms (solve included) against 95.5, 512 tiles the
+// 64x64 form.
 template <int MODE, bool UPPER>
 int sgemm_shape(hipStream_t s, int m, int n, int k, float alpha, const float *A, int lda, const float *B,
                 int ldb, float beta, float *C, int ldc, int ktri = 0)

@@ -51,12 +51,13 @@
 // (sa_dtrtri_tile) runs the same inverse items after D items that only
 // invert, so a solve on a resident factor multiplies by the same bits.
 //
-// Bound: the chain, 16.7 us a step alone on the chip (8.5 the block, 3.3 the
+// Bound: the chain, 17.6 us a step alone on the chip (8.5 the block, 3.3 the
 // stores, the look at what is prepared and its loads, 1.3 the panel product,
-// 0.9 its publication, 2.4 the diagonal update), from about 31 bulk
+// 0.9 its publication, 2.4 the diagonal update, taken apart; about 1 the waits
+// for the two write-backs), from about 31 bulk
 // workgroups on up to n = 1024, and the bulk beyond: a 1024 tile with both
-// inverses takes 336 us with 31 workgroups and 301 with 63, a 2048 tile 1534
-// with 31 and 960 with 63.  One item per block and update step (right-looking),
+// inverses takes 338 us with 31 workgroups and 302 with 63, a 2048 tile 1537
+// with 31 and 968 with 63.  One item per block and update step (right-looking),
 // each block read and written at every step and the chain's blocks handed
 // on through memory, took 43 us a step and 1357, 1056 and 907 us for a 1024
 // tile with 31, 63 and 127.
@@ -99,7 +100,7 @@ int max_bulk()
 	return v;
 }
 
-// The counters, each on a 64-byte line of its own: rows of L, then
+// The counters, 64 bytes apart (two to a 128-byte cache line): rows of L, then
 // "A(i,i) / A(i+1,i) prepared" and "D(i) done" flags, rows of W, the ticket
 // and the abort flag.
 constexpr int FLAG_STRIDE = 16;       // unsigned per line
